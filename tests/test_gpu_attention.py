@@ -142,3 +142,27 @@ def test_paged_attention_decode_nan_codes_and_bad_pages(dev, D):
     got = kv.paged_attention_decode(*args, sm_scale=0.125)
     assert_within_one_ulp(bits16(got), want, v_colmax(pool, scales, bt_bad, lens, 8))
     assert np.isnan(bf16_to_f32(bits16(got)[1, 4:8])).all()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,P,lens", [
+    (64, 8, 128, 16, [127, 128, 129, 0, 700]),     # 8 heads per block; sequence ends on and beside a unit's end
+    (32, 1, 64, 32, [513, 1, 0, 0, 255, 256]),     # 32 heads: two blocks of 16; empty sequences inside a run
+    (20, 4, 128, 48, [31, 33, 2000]),              # 5 heads per block
+    (16, 4, 64, 16, [int(v) for v in np.random.default_rng(3).integers(0, 300, 67)]),   # > 64 sequences
+    (4, 4, 128, 16, [int(v) for v in np.random.default_rng(4).integers(0, 900, 300)]),  # > 256, one head per block
+    (8, 2, 128, 16, [int(v) for v in np.random.default_rng(5).integers(0, 500, 140)]),  # whole sequences per block
+    (8, 2, 256, 16, [0, 64, 65, 1000]),
+])
+def test_paged_attention_decode_runs_and_segments(dev, Hq, Hkv, D, P, lens):
+    """The positions of all sequences are dealt to the blocks in equal runs of units (128
+    positions; 64 - 256 without matrix cores): runs that hold several sequences, sequences
+    over several runs, unit and tile edges, empty sequences, and more sequences than one wave
+    (64) or one block (256) looks through at a time.  Bound: this module's (fp32 sums)."""
+    q, pool, scales, bt, lens = make_case(Hq, Hkv, D, P, lens, seed=Hq + D + len(lens))
+    sm = 1.0 / np.sqrt(D)
+    want, werr = O.paged_attention_decode(bits16(q), pool, scales, bt, lens, sm)
+    assert werr == 0
+    got = kv.paged_attention_decode(q.to(dev), torch.from_numpy(pool).to(dev), torch.from_numpy(scales).to(dev),
+                                    torch.from_numpy(bt).to(dev), torch.from_numpy(lens).to(dev), check=True)
+    assert_within_one_ulp(bits16(got), want, v_colmax(pool, scales, bt, lens, Hq))
+    assert not bits16(got)[lens == 0].any()
