@@ -511,3 +511,66 @@ def test_ring_degree_above_sequence_lengths():
                                     causal=True, check=True, single_launch=single)
         torch.cuda.synchronize()
         assert_precision(bits16(out), want, vmax_rows(pool, scales, bt, cu, zeros, kl, Hq))
+
+
+def _f64_rows(q, pool, scales, bt, cu, qp, ranges, causal, sm):
+    """Plain float64 attention over the given key ranges ([R][B] begin / end), and max |V|."""
+    P, (n_rows, Hq, D), Hkv = pool.shape[3], q.shape, pool.shape[2]
+    out = torch.zeros(q.shape, dtype=torch.float64, device=DEV)
+    vmax = torch.zeros_like(out)
+    for b in range(len(cu) - 1):
+        t = torch.cat([torch.arange(lo[b], hi[b]) for lo, hi in ranges]).to(DEV)
+        rows = slice(int(cu[b]), int(cu[b + 1]))
+        pos = int(qp[b]) + torch.arange(rows.stop - rows.start, device=DEV)
+        kv_ = pool[bt[b, t // P].long(), :, :, t % P].view(torch.float8_e4m3fn).float().double()
+        kv_ = kv_ * scales.double()[None, :, :, None]  # [keys, 2, Hkv, D]
+        for h in range(Hq):
+            k, v = kv_[:, 0, h // (Hq // Hkv)], kv_[:, 1, h // (Hq // Hkv)]
+            s = q[rows, h].double() @ k.t().contiguous() * sm
+            if causal:
+                s.masked_fill_(t[None, :] > pos[:, None], -np.inf)
+            out[rows, h] = torch.nan_to_num(torch.softmax(s, dim=-1)) @ v
+            vmax[rows, h] = v.abs().amax(dim=0)
+    return out, vmax
+
+
+@pytest.mark.parametrize("case", ["causal", "full", "ring", "gaps", "large_scores", "bad_page"])
+@pytest.mark.parametrize("precision", ["f16", "bf16"])
+def test_wide_prefill(case, precision):
+    """The kernel with 64 rows per wave (four heads per KV head, at least a block per CU, room
+    for 4,096 positions): ragged last tiles, steps cut by range ends, ranges that follow each
+    other (walked as one) and ranges with gaps, running maxima that are outgrown again and
+    again, and a bad page.  Bound: this module's, against float64."""
+    Hq, Hkv, P = 32, 8, 48 if case == "gaps" else 16
+    n_q, q_pos0, lens = [1030, 577, 1], [0, 700, 90], [1030, 1277, 91]
+    print(f"wide prefill {case} {precision}", flush=True)
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, n_q, q_pos0, lens, seed=77)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    wide_bt = np.full((len(lens), 4096 // P + 1), -1, np.int32)
+    wide_bt[:, :bt.shape[1]] = bt
+    causal, sm = case != "full", float(np.float32(1.0 / np.sqrt(128)))
+    if case == "large_scores":
+        sm *= 12.0
+    lens = np.asarray(lens)
+    if case == "ring":
+        ranges = [(lens * r // 5, lens * (r + 1) // 5) for r in range(5)]
+    elif case == "gaps":
+        ranges = [(lens * 0 + 5, lens // 3), (lens // 2, lens - 7)]
+    else:
+        ranges = [(lens * 0, lens)]
+    q, pool, scales, bt = q.to(DEV), t(pool), t(scales), t(wide_bt)
+    if case == "bad_page":
+        bt[1, 20] = pool.shape[0]
+        with pytest.raises(ValueError, match="block table"):
+            kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, t(np.array([r[0] for r in ranges], np.int32)),
+                                    t(np.array([r[1] for r in ranges], np.int32)), check=True, precision=precision)
+        ranges = [(np.array([0, 0, 0]), np.array([lens[0], 20 * P, lens[2]])),
+                  (np.array([0, 21 * P, 0]), np.array([0, lens[1], 0]))]
+        got = kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, t(np.zeros((1, 3), np.int32)),
+                                      t(lens[None].astype(np.int32)), precision=precision)
+    else:
+        got = kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, t(np.array([r[0] for r in ranges], np.int32)),
+                                      t(np.array([r[1] for r in ranges], np.int32)), causal=causal, sm_scale=sm,
+                                      check=True, precision=precision)
+    want, vmax = _f64_rows(q, pool, scales, bt, cu, qp, ranges, causal, sm)
+    assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy(), precision)

@@ -29,9 +29,14 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function",
 ]
-# per-file options: under this machine scheduler the fused append's loads issue in longer
-# clauses (0.5-0.8% less time per 32-layer x 74,902-token append on MI355X, same codes)
-FILE_FLAGS = {"zx_append_fused.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"]}
+# per-file options:
+# * append: under this machine scheduler the fused append's loads issue in longer clauses
+#   (0.5-0.8% less time per 32-layer x 74,902-token append on MI355X, same codes);
+# * prefill: matrix results in vector registers.  By default a kernel that may use more than
+#   256 registers takes them in accumulation registers, and the 64-row kernel copied every
+#   score out again (64 moves per step, and spills).
+FILE_FLAGS = {"zx_append_fused.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],
+              "zx_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def hipcc() -> str:

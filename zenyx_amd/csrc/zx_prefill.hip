@@ -654,6 +654,559 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
   if (e && a.err) atomicOr(a.err, e);
 }
 
+// ---------------------------------------------------------------- 64 rows per wave
+//
+// The same problem for large prefills that write their rows as bf16 (no running output):
+// 64 query rows per wave (two groups of 32), 32x32x16 matrix tiles, one wave per SIMD with
+// the registers of two.  The kernel above is bound by latencies that two waves per SIMD do
+// not hide and reads every K/V operand from LDS for 32 rows (LDS active 58% of the cycles);
+// with 64 rows the operand traffic halves, and one instruction stream is laid out by hand:
+//   * S^T of step j (32 matrix instructions) beside the decode and store of step j + 1's K
+//     and V and the weights of the step's first 32 keys;
+//   * P.V of step j - 1 beside the weights of the last 32 keys and the packing of P, each
+//     chunk of P right after the products that read its predecessor.
+// A matrix instruction leaves the vector unit about half of its time, so the two kinds of
+// work add up to what the vector unit can issue (a step of 64 keys: ~2,000 + ~2,000 cycles
+// measured for the two halves, 1,107 + 1,107 of them matrix time).
+// No running maximum is computed in these steps: the weights are taken under the maxima the
+// rows have, and only if a lane's sum shows that a score has outgrown them (2^PF_LAZY, as
+// above), or where masks apply or a row has no key yet, the step's S^T is made again and
+// the maxima are looked at (K has three buffers in LDS for that, V^T four: a wave may be one
+// step ahead of another).  Looking at the maxima in every step cost 12% (2.17 against 2.10
+// ms); leaving its exponentials in one half of the step, with scalar page lookups between
+// the halves, 2.22 ms.
+// 4 x 8,192 causal, Hq 32 / Hkv 8 (one launch): 2.31 -> 2.18 ms on one box (2.10 on another,
+// 1,045 TFLOP/s); 2 x 4,096 not causal 620 -> 572 us; 2,048 rows on 8,192 cached 387 -> 365 us.
+typedef _Float16 pw_f16x2 __attribute__((ext_vector_type(2)));
+typedef float att_f32x16 __attribute__((ext_vector_type(16)));
+constexpr int PW_ROWS = 64;                   // query rows per wave and per block
+constexpr int PW_KBYTES = PF_KEYS * PF_KROW;  // one K buffer (of 3)
+constexpr int PW_VBYTES = 128 * PF_VROW;      // one V^T buffer (of 4)
+
+__device__ __forceinline__ att_f32x16 pw_mfma_bf16(att_u32x4 a, att_u32x4 b, att_f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf16x8, a), __builtin_bit_cast(att_bf16x8, b),
+                                                 c, 0, 0, 0);
+}
+__device__ __forceinline__ att_f32x16 pw_mfma_f16(att_u32x4 a, att_u32x4 b, att_f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(att_f16x8, a), __builtin_bit_cast(att_f16x8, b), c,
+                                                0, 0, 0);
+}
+
+// V^T in LDS: row 8 (c % 16) + c / 16 holds channel c, so that a store of a wave (lanes'
+// channels 16 apart) falls on rows next to each other and no swizzle is needed: the operand
+// reads are one base plus constants.  Within a row the 64 keys are in the order in which
+// the S^T tiles leave them: chunk kc (16 keys), lane half hl, element j (8) is key
+// 16 kc + 8 (j / 4) + 4 hl + j % 4, at byte 32 kc + 16 hl + 2 j.
+__device__ __forceinline__ int pw_vslot_byte(int c, int key) {
+  const int kc = key >> 4, y = key & 15;
+  return (8 * (c & 15) + (c >> 4)) * PF_VROW + 32 * kc + 16 * ((y >> 2) & 1) + 2 * (4 * (y >> 3) + (y & 3));
+}
+
+template <int PM>
+__global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(PrefillArgs a) {
+  constexpr bool F16 = PM == PF_P_F16;
+  constexpr int D = 128;
+  constexpr int G = 4, QT = PW_ROWS;  // query heads (one per wave) and rows per block
+  const int n_hg = a.n_q_heads / G;
+  const int64_t per_rank = (int64_t)n_hg * a.n_seqs;
+  const int64_t qt_rev = (int64_t)blockIdx.x / per_rank;
+  const int rem = (int)((int64_t)blockIdx.x - qt_rev * per_rank);
+  const int hg = rem % n_hg, b = rem / n_hg;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane & 31, hl = lane >> 5;
+  const int grp = a.n_q_heads / a.n_kv_heads;
+  const int hq = hg * G + wave;
+  const int h = (hg * G) / grp;
+  const int32_t cq0 = a.cu_q[b], cq1 = a.cu_q[b + 1], qp0_32 = a.q_pos0[b];
+  const int32_t kb0 = a.kv_begin[b], ke0 = a.kv_end[b];
+  const float sk = a.scales[h], sv = a.scales[a.n_kv_heads + h];
+  // (together: see the kernel above)
+  asm volatile("" ::"s"(cq0), "s"(cq1), "s"(qp0_32), "s"(kb0), "s"(ke0), "s"(sk), "s"(sv));
+  const int64_t qp0 = qp0_32;
+  const int64_t q_lo = cq0;
+  const int n_qb = cq1 - cq0;
+  const int64_t row0_64 = ((int64_t)a.n_qt - 1 - qt_rev) * QT;
+  if (row0_64 >= n_qb) return;
+  const int row0_blk = (int)row0_64;
+  const int wrow0 = row0_blk;  // all waves: the same rows of their own head
+  const int64_t page_bytes = 2LL * a.n_kv_heads * a.page_size * D;
+  const int64_t head_off = (int64_t)h * a.page_size * D;
+  const int64_t v_off = (int64_t)a.n_kv_heads * a.page_size * D;
+  const int32_t *bt = a.bt + (int64_t)b * a.max_blocks;
+  int32_t e = 0;
+  if (qt_rev == 0 && (int64_t)a.n_qt * QT < n_qb) e |= ZX_KERR_POS_RANGE;
+  const int kmax = a.max_blocks * a.page_size;
+  const int last_row = min(row0_blk + QT, n_qb) - 1;
+  // Range r of this sequence: keys [kb, ke) (ke clipped to the block table), walked in
+  // 64-key steps from s_first (kb rounded down to a 16-key tile) while below ke_blk (ke, or
+  // the block's last causal key + 1).  All block-uniform.  Ranges that follow each other
+  // without a gap (the shards of a ring) are walked as one.
+  struct Range {
+    int kb, ke, s_first, ke_blk;
+  };
+  __shared__ int32_t rtab[2][PF_RTAB];
+  const int n_tab = a.n_ranges > 1 ? min(a.n_ranges, PF_RTAB) : 0;
+  int n_ranges = a.n_ranges, ke_one = ke0;
+  if (n_tab) {  // block-uniform
+    bool gap = a.n_ranges > PF_RTAB;
+    for (int r = threadIdx.x; r < n_tab; r += PF_THREADS) {
+      const int64_t i = (int64_t)r * a.n_seqs + b;
+      const int32_t kbr = a.kv_begin[i], ker = a.kv_end[i];
+      rtab[0][r] = kbr;
+      rtab[1][r] = ker;
+      gap |= kbr < 0 || ker < kbr || (r > 0 && a.kv_end[i - a.n_seqs] != kbr);
+    }
+    if (!__syncthreads_or(gap)) {
+      n_ranges = 1;
+      ke_one = __builtin_amdgcn_readfirstlane(rtab[1][n_tab - 1]);
+    }
+  }
+  auto range = [&](int r) -> Range {
+    Range g;
+    int32_t kbr, ker;
+    if (r == 0) {
+      kbr = kb0;
+      ker = ke_one;
+    } else if (r < n_tab) {
+      kbr = __builtin_amdgcn_readfirstlane(rtab[0][r]);
+      ker = __builtin_amdgcn_readfirstlane(rtab[1][r]);
+    } else {
+      const int64_t i = (int64_t)r * a.n_seqs + b;
+      kbr = a.kv_begin[i];
+      ker = a.kv_end[i];
+    }
+    g.kb = kbr > 0 ? kbr : 0;
+    g.ke = ker;
+    if (g.ke > kmax) {
+      e |= ZX_KERR_POS_RANGE;
+      g.ke = kmax;
+    }
+    g.ke_blk = a.causal ? (int)max((int64_t)-1, min((int64_t)g.ke, qp0 + last_row + 1)) : g.ke;
+    g.s_first = (g.kb / 16) * 16;
+    return g;
+  };
+  // the first range with a step at or after r (n_ranges if none)
+  auto next_range = [&](int r, Range &g) -> int {
+    for (; r < n_ranges; ++r) {
+      g = range(r);
+      if (g.s_first < g.ke_blk) return r;
+    }
+    return n_ranges;
+  };
+  Range g;
+  int rc = next_range(0, g);
+  __shared__ __attribute__((aligned(16))) uint8_t kst[3 * PW_KBYTES];
+  __shared__ __attribute__((aligned(16))) uint8_t vtl[4 * PW_VBYTES];
+
+  const float qs = sk * a.sm_log2e;
+  const float vscale = sv;
+  att_f32x16 o[2][4];  // [rg][ct]: channels 32 ct + 8 t + 4 hl ..+4 of row 32 rg + n
+  float m[2], l[2];
+#pragma unroll
+  for (int rg = 0; rg < 2; ++rg) {
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[rg][ct][i] = 0.0f;
+    m[rg] = -INFINITY;
+    l[rg] = 0.0f;
+  }
+  const float p_shift = F16 ? PF_F16_SHIFT : 0.0f;
+  const int kp2 = threadIdx.x >> 3, g8 = threadIdx.x & 7;
+  const int kk0 = 2 * kp2;
+  struct Codes {
+    att_u32x4 k[2], v[2];
+  };
+  // Where the codes of 64 steps' tiles are (this wave's 16-key tile of each step): lane i
+  // holds step base + i's byte offset in the pool and its bytes of valid rows, so that a
+  // step costs three readlanes instead of a page lookup and its scalar arithmetic.
+  uint32_t tab_lo = 0, tab_hi = 0;
+  int tab_n = 0;
+  auto fill_table = [&](int base) {
+    const int64_t tp = (int64_t)g.s_first + (int64_t)(base + lane) * PF_KEYS + 16 * wave;
+    const int n_live = (int)max((int64_t)0, min((int64_t)16, g.ke - tp));
+    const uint32_t tc = n_live ? (uint32_t)tp : 0u;
+    const uint32_t bi = pf_page_of(a, tc);
+    const int64_t page = n_live && g.s_first + (int64_t)(base + lane) * PF_KEYS < g.ke_blk ? bt[bi] : 0;
+    const bool ok = page >= 0 && page < a.n_pages;
+    e |= ok ? 0 : ZX_KERR_PAGE_RANGE;
+    const uint64_t off =
+        ok ? (uint64_t)(page * page_bytes + head_off + (int64_t)(tc - bi * (uint32_t)a.page_size) * D) : 0;
+    tab_lo = (uint32_t)off;
+    tab_hi = (uint32_t)(off >> 32);
+    tab_n = ok ? n_live * D : 0;
+  };
+  const int ld_off = (kk0 & 15) * D + 16 * g8;
+  // K and V codes of step i of the range into registers (past its end: nothing is read)
+  auto issue_step = [&](int i, Codes &c) {
+    const uint64_t off = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)tab_lo, i & 63) |
+                         (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)tab_hi, i & 63) << 32;
+    const int nrec = __builtin_amdgcn_readlane(tab_n, i & 63);
+    const uint8_t *src = a.pool + off;
+    const __amdgpu_buffer_rsrc_t rk =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(src), (short)0, nrec, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(src + v_off), (short)0, nrec, 0x00020000);
+    c.k[0] = __builtin_amdgcn_raw_buffer_load_b128(rk, ld_off, 0, 0);
+    c.k[1] = __builtin_amdgcn_raw_buffer_load_b128(rk, ld_off + D, 0, 0);
+    c.v[0] = __builtin_amdgcn_raw_buffer_load_b128(rv, ld_off, 0, 0);
+    c.v[1] = __builtin_amdgcn_raw_buffer_load_b128(rv, ld_off + D, 0, 0);
+  };
+  const int kst_off = kk0 * PF_KROW + 32 * g8;
+  const int vst_off = pw_vslot_byte(16 * g8, kk0);
+  auto store_k = [&](int kbuf, int j, const Codes &c) {
+    uint32_t kb8[8];
+    decode16_bf16(make_uint4(c.k[j].x, c.k[j].y, c.k[j].z, c.k[j].w), kb8);
+    uint4 *kd = reinterpret_cast<uint4 *>(&kst[kbuf + kst_off + j * PF_KROW]);
+    kd[0] = make_uint4(kb8[0], kb8[1], kb8[2], kb8[3]);
+    kd[1] = make_uint4(kb8[4], kb8[5], kb8[6], kb8[7]);
+  };
+  // V^T of channels 16 g8 + 4 q ..+4 (q < 4): two code words of each key
+  auto store_v = [&](int vbuf, int q, const Codes &c) {
+    uint32_t v0[2], v1[2];
+    const int w0 = (int)c.v[0][q], w1 = (int)c.v[1][q];
+    if constexpr (F16) {
+      v0[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 1.0f, false));
+      v0[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w0, 1.0f, true));
+      v1[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 1.0f, false));
+      v1[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w1, 1.0f, true));
+    } else {
+      v0[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, false));
+      v0[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w0, 1.0f, true));
+      v1[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, false));
+      v1[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w1, 1.0f, true));
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      uint8_t *row = &vtl[vbuf + vst_off + (4 * q + 2 * p) * 8 * PF_VROW];
+      *reinterpret_cast<uint32_t *>(row) = __builtin_amdgcn_perm(v1[p], v0[p], 0x05040100u);
+      *reinterpret_cast<uint32_t *>(row + 8 * PF_VROW) = __builtin_amdgcn_perm(v1[p], v0[p], 0x07060302u);
+    }
+  };
+
+  att_u32x4 qa[2][8];
+#pragma unroll
+  for (int rg = 0; rg < 2; ++rg) {
+    const int r = min(wrow0 + 32 * rg + n, n_qb - 1);  // rows past the last repeat it, and are not stored
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      qa[rg][c] =
+          *reinterpret_cast<const att_u32x4 *>(a.q + ((q_lo + r) * a.n_q_heads + hq) * D + c * 16 + hl * 8);
+  }
+  Codes ca, cb;
+  if (rc < n_ranges) {
+    fill_table(0);
+    issue_step(0, ca);
+    issue_step(1, cb);
+  }
+  bool all_ok;
+  {
+    bool bad = false;
+    for (int r = 0; r < n_ranges; ++r) {
+      const Range w = range(r);
+      if (w.s_first >= w.ke) continue;
+      const int p_lo = (int)pf_page_of(a, (uint32_t)w.s_first), p_hi = (int)pf_page_of(a, (uint32_t)(w.ke - 1));
+      for (int pi = p_lo + (int)threadIdx.x; pi <= p_hi; pi += PF_THREADS) {
+        const int64_t pg = bt[pi];
+        bad |= pg < 0 || pg >= a.n_pages;
+      }
+    }
+    all_ok = !__syncthreads_or(bad);
+  }
+  auto tile_ok = [&](int tp, int ke) -> bool {
+    if (tp >= ke) return false;
+    if (all_ok) return true;
+    const int64_t page = bt[pf_page_of(a, (uint32_t)tp)];
+    return page >= 0 && page < a.n_pages;
+  };
+  att_u32x4 ph[2][4];  // [rg][kc] P^T as 16-bit pairs
+  const int k_lane = n * PF_KROW + hl * 16;
+  const int v_lane = n * PF_VROW + hl * 16;
+  auto ld_k = [&](int kbuf, int t) -> att_u32x4 {  // t = 8 KT + c
+    return *reinterpret_cast<const att_u32x4 *>(&kst[kbuf + k_lane + (t >> 3) * 32 * PF_KROW + (t & 7) * 32]);
+  };
+  auto ld_v = [&](int vbuf, int t) -> att_u32x4 {  // t = 4 kc + ct
+    return *reinterpret_cast<const att_u32x4 *>(&vtl[vbuf + v_lane + (t & 3) * 32 * PF_VROW + (t >> 2) * 32]);
+  };
+  constexpr int FD = 3;  // operand reads ahead
+  // the last key position a row may see, and the last step start at which every row of this
+  // wave sees every key (of a range)
+  auto row_lim = [&](int r) {
+    return a.causal ? (int)min(max(qp0 + min(r, n_qb - 1), (int64_t)-1), (int64_t)INT32_MAX) : INT32_MAX;
+  };
+  const int lim[2] = {row_lim(wrow0 + n), row_lim(wrow0 + 32 + n)};
+  const int s_full = all_ok && qs >= 0.0f ? row_lim(wrow0) - (PF_KEYS - 1) : -1;
+  att_u32x4 kf[FD + 1], vf[FD + 1];
+  auto pv_tile = [&](int t) {
+    const att_u32x4 av = vf[t % (FD + 1)];
+    const int kc = t >> 2, ct = t & 3;
+#pragma unroll
+    for (int rg = 0; rg < 2; ++rg) {
+      if constexpr (F16) o[rg][ct] = pw_mfma_f16(av, ph[rg][kc], o[rg][ct]);
+      else o[rg][ct] = pw_mfma_bf16(av, ph[rg][kc], o[rg][ct]);
+    }
+  };
+  using Scores = att_f32x16[2][2];  // [rg][KT]
+  // word w of the weights of key chunk kc as 16-bit pairs, and the chunk's sum
+  auto pack_p = [&](const Scores &s, float (&ls)[2][2], int kc, int w) {
+#pragma unroll
+    for (int rg = 0; rg < 2; ++rg) {
+      const int i = 8 * (kc & 1) + 2 * w;
+      const float x = s[rg][kc >> 1][i], y = s[rg][kc >> 1][i + 1];
+      // (a scalar first: with this compiler __builtin_bit_cast of a vector's element reads
+      // element 0)
+      const uint32_t pw = F16 ? pack_f16(x, y) : pack_bf16(x, y);
+      ph[rg][kc][w] = pw;
+      if constexpr (F16)
+        ls[rg][w & 1] = __builtin_amdgcn_fdot2(__builtin_bit_cast(pw_f16x2, pw), pw_f16x2{(_Float16)1, (_Float16)1},
+                                               ls[rg][w & 1], false);
+      else
+        ls[rg][w & 1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(att_bf2, pw),
+                                                        __builtin_bit_cast(att_bf2, 0x3F803F80u), ls[rg][w & 1], false);
+    }
+  };
+  // keeps a chunk's weights where they are made: beside the products, not sunk past them
+  auto pin_p = [&](float (&ls)[2][2], int kc) {
+    asm volatile("" : "+v"(ph[0][kc]), "+v"(ph[1][kc]), "+v"(ls[0][0]), "+v"(ls[0][1]), "+v"(ls[1][0]), "+v"(ls[1][1]));
+  };
+  auto qk_tile = [&](Scores &s, int t) {  // t = 8 KT + c
+    const int KT = t >> 3, c = t & 7;
+#pragma unroll
+    for (int rg = 0; rg < 2; ++rg) {
+      if (c == 0) {
+        att_f32x16 z;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+        s[rg][KT] = pw_mfma_bf16(kf[t % (FD + 1)], qa[rg][c], z);
+      } else {
+        s[rg][KT] = pw_mfma_bf16(kf[t % (FD + 1)], qa[rg][c], s[rg][KT]);
+      }
+    }
+  };
+  // exponents, then weights, of elements i0 ..+n_e of key tile KT (a weight right after its
+  // own exponent would wait for it)
+  auto weights = [&](Scores &s, int KT, int i0, int n_e, float q, const float (&cst)[2]) {
+    float x[2][8];
+#pragma unroll
+    for (int rg = 0; rg < 2; ++rg)
+#pragma unroll
+      for (int u = 0; u < n_e; ++u) x[rg][u] = __builtin_fmaf(s[rg][KT][i0 + u], q, cst[rg]);
+#pragma unroll
+    for (int u = 0; u < n_e; ++u) asm volatile("" : "+v"(x[0][u]), "+v"(x[1][u]));
+#pragma unroll
+    for (int rg = 0; rg < 2; ++rg)
+#pragma unroll
+      for (int u = 0; u < n_e; ++u) s[rg][KT][i0 + u] = __builtin_amdgcn_exp2f(x[rg][u]);
+  };
+  constexpr float L_MOST = F16 ? 32768.0f : 256.0f;  // 2^(p_shift + PF_LAZY)
+  float cst[2] = {-INFINITY, -INFINITY};
+  bool m_ok = false;  // every row of the wave has a running maximum
+
+  while (rc < n_ranges) {  // a range: its steps j = 0 .. n_steps - 1
+    store_k(0, 0, ca);
+    store_k(0, 1, ca);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) store_v(0, q, ca);
+    // the V^T buffer that the first step's (empty) P.V reads
+    for (int i = threadIdx.x; i < PW_VBYTES / 16; i += PF_THREADS)
+      *reinterpret_cast<uint4 *>(&vtl[3 * PW_VBYTES + 16 * i]) = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+    for (int rg = 0; rg < 2; ++rg)
+#pragma unroll
+      for (int kc = 0; kc < 4; ++kc) ph[rg][kc] = att_u32x4{0u, 0u, 0u, 0u};
+    __syncthreads();
+    int kbuf = 0, vrd = 3 * PW_VBYTES, vnext = PW_VBYTES;
+#pragma unroll
+    for (int t = 0; t < FD; ++t) kf[t] = ld_k(0, t);
+    const int s_hi = min(g.ke - PF_KEYS, s_full);
+    const int n_steps = (g.ke_blk - g.s_first + PF_KEYS - 1) / PF_KEYS;
+    for (int j = 0; j < n_steps;) {
+      // the steps that every row of the wave sees whole, under the running maxima it has
+      int kb_n = kbuf == 2 * PW_KBYTES ? 0 : kbuf + PW_KBYTES;
+      float ls[2][2];
+      bool grown = false;
+      auto next_step = [&]() {
+#pragma unroll
+        for (int rg = 0; rg < 2; ++rg) l[rg] += ls[rg][0] + ls[rg][1];
+        kbuf = kb_n;
+        kb_n = kbuf == 2 * PW_KBYTES ? 0 : kbuf + PW_KBYTES;
+        vrd = vrd == 3 * PW_VBYTES ? 0 : vrd + PW_VBYTES;
+        vnext = vnext == 3 * PW_VBYTES ? 0 : vnext + PW_VBYTES;
+        ++j;
+      };
+      while (m_ok && j < n_steps) {
+        const int s0 = g.s_first + j * PF_KEYS;
+        if (s0 < g.kb || s0 > s_hi) break;
+        if (((j + 2) & 63) == 0) fill_table(j + 2);
+        ls[0][0] = ls[0][1] = ls[1][0] = ls[1][1] = 0.0f;
+        Scores s;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+          if (t + FD < 16) kf[(t + FD) % (FD + 1)] = ld_k(kbuf, t + FD);
+          else vf[t + FD - 16] = ld_v(vrd, t + FD - 16);
+          qk_tile(s, t);
+          if (t == 0) store_k(kb_n, 0, cb);
+          if (t == 2) store_k(kb_n, 1, cb);
+          if (t >= 3 && t < 7) store_v(vnext, t - 3, cb);
+          if (t >= 9 && t < 14) weights(s, 0, 3 * (t - 9), 3, qs, cst);
+          if (t == 14) weights(s, 0, 15, 1, qs, cst);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+          if (t + FD < 16) vf[(t + FD) % (FD + 1)] = ld_v(vrd, t + FD);
+          else kf[t + FD - 16] = ld_k(kb_n, t + FD - 16);
+          pv_tile(t);
+          if (t == 0) issue_step(j + 2, cb);
+          if (t < 8) weights(s, 1, 2 * t, 2, qs, cst);
+          if (t >= 4) {  // P of kc is free after tile 4 kc + 3
+            pack_p(s, ls, (t >> 2) - 1, t & 3);
+            if ((t & 3) == 3) pin_p(ls, (t >> 2) - 1);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) pack_p(s, ls, 3, w);
+        pin_p(ls, 3);
+        const bool big = fmaxf(fmaxf(ls[0][0], ls[0][1]), fmaxf(ls[1][0], ls[1][1])) > L_MOST;
+        if (__builtin_amdgcn_ballot_w64(big)) {
+          grown = true;
+          break;
+        }
+        next_step();
+      }
+      if (j >= n_steps) break;
+      const int s0 = g.s_first + j * PF_KEYS;
+      if (!grown) {
+        if (((j + 2) & 63) == 0) fill_table(j + 2);
+        store_k(kb_n, 0, cb);
+        store_k(kb_n, 1, cb);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) store_v(vnext, q, cb);
+#pragma unroll
+        for (int t = 0; t < FD; ++t) vf[t] = ld_v(vrd, t);
+        __syncthreads();
+        issue_step(j + 2, cb);
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+          if (t + FD < 16) vf[(t + FD) % (FD + 1)] = ld_v(vrd, t + FD);
+          pv_tile(t);
+        }
+      }
+      {
+        const bool full = s0 >= g.kb && s0 <= s_hi;
+        // the step with its running maxima looked at and the masks applied: the first step, the
+        // steps that cross a boundary, and one whose weights outgrew the maxima (its S^T made
+        // again; this step's K is still in LDS)
+        Scores s;
+#pragma unroll
+        for (int t = 0; t < FD; ++t) kf[t] = ld_k(kbuf, t);
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+          if (t + FD < 16) kf[(t + FD) % (FD + 1)] = ld_k(kbuf, t + FD);
+          qk_tile(s, t);
+        }
+#pragma unroll
+        for (int t = 0; t < FD; ++t) kf[t] = ld_k(kb_n, t);
+        float qe = qs;
+        if (!full) {  // scores times qs, -inf where the (row, key) does not count
+          uint32_t tk = 0;
+#pragma unroll
+          for (int T = 0; T < 4; ++T) tk |= tile_ok(s0 + 16 * T, g.ke) ? 1u << T : 0u;
+#pragma unroll
+          for (int i = 0; i < 32; ++i) {
+            const int kp = s0 + 8 * (i >> 2) + 4 * hl + (i & 3);
+            const bool in = ((tk >> (i >> 3)) & 1u) != 0 && kp >= g.kb && kp < g.ke;
+#pragma unroll
+            for (int rg = 0; rg < 2; ++rg)
+              s[rg][i >> 4][i & 15] = in && kp <= lim[rg] ? s[rg][i >> 4][i & 15] * qs : -INFINITY;
+          }
+          qe = 1.0f;
+        }
+        bool grow_any = false, ok = true;
+        float alpha[2];
+#pragma unroll
+        for (int rg = 0; rg < 2; ++rg) {
+          float mx = -INFINITY, x, y;
+#pragma unroll
+          for (int i = 0; i < 32; i += 2) mx = fmaxf(fmaxf(mx, s[rg][i >> 4][i & 15]), s[rg][i >> 4][(i & 15) + 1]);
+          xrow_pair32(mx * qe, x, y);
+          const float w = fmaxf(x, y);
+          const bool grow = w > m[rg] + PF_LAZY;
+          const float mn = grow ? w : m[rg];
+          const float ms = mn == -INFINITY ? 0.0f : mn;  // a row with no key yet keeps p = 0
+          alpha[rg] = grow ? __builtin_amdgcn_exp2f(m[rg] - ms) : 1.0f;
+          grow_any |= grow;
+          ok &= mn != -INFINITY;
+          m[rg] = mn;
+          l[rg] *= alpha[rg];
+          cst[rg] = p_shift - ms;
+          ls[rg][0] = ls[rg][1] = 0.0f;
+        }
+        m_ok = __builtin_amdgcn_ballot_w64(!ok) == 0;
+#pragma unroll
+        for (int KT = 0; KT < 2; ++KT)
+#pragma unroll
+          for (int i = 0; i < 16; i += 8) weights(s, KT, i, 8, qe, cst);
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc)
+#pragma unroll
+          for (int w = 0; w < 4; ++w) pack_p(s, ls, kc, w);
+          // rescale O only when some row's maximum was raised
+        if (__builtin_amdgcn_ballot_w64(grow_any)) {
+#pragma unroll
+          for (int rg = 0; rg < 2; ++rg)
+#pragma unroll
+            for (int ct = 0; ct < 4; ++ct) o[rg][ct] *= alpha[rg];
+        }
+      }
+      next_step();
+    }
+    // P.V of the last step
+#pragma unroll
+    for (int t = 0; t < FD; ++t) vf[t] = ld_v(vrd, t);
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      if (t + FD < 16) vf[(t + FD) % (FD + 1)] = ld_v(vrd, t + FD);
+      pv_tile(t);
+    }
+    rc = next_range(rc + 1, g);
+    if (rc < n_ranges) {
+      fill_table(0);
+      issue_step(0, ca);
+      issue_step(1, cb);
+      __syncthreads();
+    }
+  }
+
+  // rows: normalise; store.  O^T row 32 ct + 8 t + 4 hl + i is channel
+  // 16 (4 hl + i) + 4 ct + t: 16 channels in a row per i.
+#pragma unroll
+  for (int rg = 0; rg < 2; ++rg) {
+    const int r = wrow0 + 32 * rg + n;
+    float lx, ly;
+    xrow_pair32(l[rg], lx, ly);
+    const float lt = lx + ly;
+    if (r >= n_qb) continue;
+    const float inv = lt > 0.0f ? vscale / lt : 0.0f;  // V's dequant scale applied once, here
+    uint4 *out = reinterpret_cast<uint4 *>(a.out + ((q_lo + r) * a.n_q_heads + hq) * D + 64 * hl);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t w[8];
+#pragma unroll
+      for (int ct = 0; ct < 4; ++ct) {
+        w[2 * ct] = pack_bf16(o[rg][ct][i] * inv, o[rg][ct][4 + i] * inv);
+        w[2 * ct + 1] = pack_bf16(o[rg][ct][8 + i] * inv, o[rg][ct][12 + i] * inv);
+      }
+      out[2 * i] = make_uint4(w[0], w[1], w[2], w[3]);
+      out[2 * i + 1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+  }
+  if (e && a.err) atomicOr(a.err, e);
+}
+
 }  // namespace zx
 
 using namespace zx;
@@ -728,13 +1281,26 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
     a.p_shift = shift;
     a.p_magic = (uint32_t)(((1ULL << (31 + shift)) + page_size - 1) / page_size);
   }
-  const int QT = 32 * 4 / G;
+  const int pm = (flags & ZX_PREFILL_EXACT_P) ? PF_P_EXACT : ((flags & ZX_PREFILL_FAST_P) ? PF_P_BF16 : PF_P_F16);
+  // 64 rows per wave where nothing is merged, four query heads share a KV head, there is a
+  // block per CU and contexts can be long: its blocks start and end more slowly (3 x 500-2,000
+  // rows of new sequences: 102 against 90 us; 4 x 512 rows on 8,192 cached: 329 against 346),
+  // one or two heads per KV head gained nothing (2 x 4,096: 150 against 140, 175 against 175),
+  // and the exact mode's second set of weights does not fit its registers.
+  const bool wide = G == 4 && !(flags & ZX_PREFILL_MERGE) && pm != PF_P_EXACT &&
+                    (int64_t)max_blocks * page_size >= 4096 &&
+                    ceil_div(max_q_per_seq, PW_ROWS) * (n_q_heads / G) * n_seqs >= num_cus();
+  const int QT = wide ? PW_ROWS : 32 * 4 / G;
   a.n_qt = (int32_t)ceil_div(max_q_per_seq, QT);
   const int64_t n_blocks = (int64_t)a.n_qt * (n_q_heads / G) * n_seqs;
   ZX_REQUIRE(n_blocks < (1LL << 31), "paged_attention_prefill: too many query tiles or sequences");
   const dim3 grid((unsigned)n_blocks);
   hipStream_t st = as_stream(stream);
-  const int pm = (flags & ZX_PREFILL_EXACT_P) ? PF_P_EXACT : ((flags & ZX_PREFILL_FAST_P) ? PF_P_BF16 : PF_P_F16);
+  if (wide) {
+    if (pm == PF_P_F16) paged_prefill_wide_kernel<PF_P_F16><<<grid, PF_THREADS, 0, st>>>(a);
+    else paged_prefill_wide_kernel<PF_P_BF16><<<grid, PF_THREADS, 0, st>>>(a);
+    return check_launch("paged_prefill_wide");
+  }
   switch (G * 4 + pm) {
 #define ZX_PF_CASE(g, m) \
   case g * 4 + m: paged_prefill_mfma_kernel<g, m><<<grid, PF_THREADS, 0, st>>>(a); break;
