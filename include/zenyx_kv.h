@@ -430,6 +430,29 @@ int zx_paged_attention_ring(const uint16_t *q, int64_t n_q, const int32_t *cu_q,
                             int32_t n_seqs, int32_t max_q_per_seq, int32_t causal, float sm_scale, int32_t flags,
                             float *o_acc, float *lse2, uint16_t *out, int32_t *err, zx_stream_t stream);
 
+/* zx_paged_attention_ring with room for partial results (ABI version 8): a call with few
+ * query tiles (a chunk of a prompt, a few speculative tokens) whose rows go to out as bf16
+ * without merging lets several blocks share a tile's keys and combines their parts, within
+ * the tolerance of a ring's steps.  workspace: zx_paged_attention_ring_workspace_bytes()
+ * device bytes (16-byte aligned) for the same arguments; 0 when the call is not cut, and a
+ * smaller or NULL workspace runs it uncut.  n_ranges = 1 is one range per sequence. */
+size_t zx_paged_attention_ring_workspace_bytes(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int32_t page_size,
+                                               int32_t max_blocks, int32_t n_seqs, int32_t max_q_per_seq,
+                                               int32_t causal, int32_t flags);
+int zx_paged_attention_ring_ws(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int32_t *q_pos0,
+                               int32_t n_q_heads, const uint8_t *pool, int64_t n_pages, int32_t n_kv_heads,
+                               int32_t head_dim, int32_t page_size, const float *scales, const int32_t *block_tables,
+                               int32_t max_blocks, const int32_t *kv_begin, const int32_t *kv_end, int32_t n_ranges,
+                               int32_t n_seqs, int32_t max_q_per_seq, int32_t causal, float sm_scale, int32_t flags,
+                               float *o_acc, float *lse2, uint16_t *out, int32_t *err, void *workspace,
+                               size_t workspace_bytes, zx_stream_t stream);
+
+/* Key ranges of a ring's shards (ABI version 8): for r < degree, kv_begin[r * row_stride + b]
+ * = floor(r kv_len[b] / degree) and kv_end[...] = floor((r + 1) kv_len[b] / degree), all
+ * device int32, row_stride >= n_seqs. */
+int zx_ring_shard_bounds(const int32_t *kv_len, int32_t n_seqs, int32_t degree, int32_t row_stride,
+                         int32_t *kv_begin, int32_t *kv_end, zx_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

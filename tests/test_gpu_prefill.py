@@ -574,3 +574,56 @@ def test_wide_prefill(case, precision):
                                       check=True, precision=precision)
     want, vmax = _f64_rows(q, pool, scales, bt, cu, qp, ranges, causal, sm)
     assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy(), precision)
+
+
+@pytest.mark.parametrize("Hq,Hkv,P,n_q,q_pos0,causal,precision", [
+    (32, 8, 16, [5, 1, 40], [1500, 600, 2100], True, "f16"),   # several parts; sequences of different lengths
+    (8, 2, 16, [33], [1023], True, "exact"),                   # a part per 8 steps, tiles of 32 rows and 1
+    (4, 4, 48, [130, 3], [2000, 12], True, "bf16"),            # one head per KV head; a sequence with keys for one part
+    (6, 3, 32, [17, 64], [0, 900], False, "f16"),              # every row sees every key
+])
+def test_prefill_in_parts(Hq, Hkv, P, n_q, q_pos0, causal, precision):
+    """Calls with few query tiles: several blocks share a tile's keys and their parts are
+    combined; with a ring's contiguous shards and with a gap between two ranges.  Rows beyond
+    max_q_per_seq stay unwritten.  Bound: this module's, against float64 (the combination is
+    an average under the same weights in fp32, far below it)."""
+    lens = np.asarray([p + n for p, n in zip(q_pos0, n_q)])
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, n_q, q_pos0, lens.tolist(), seed=5 * Hq + P)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    q, pool, scales, bt = q.to(DEV), t(pool), t(scales), t(bt)
+    sm = float(np.float32(1.0 / np.sqrt(128)))
+    for ranges in ([(lens * r // 3, lens * (r + 1) // 3) for r in range(3)], [(lens * 0 + 3, lens // 3), (lens // 2, lens)]):
+        kb, ke = (t(np.array([r[i] for r in ranges], np.int32)) for i in (0, 1))
+        got = kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, kb, ke, causal=causal, sm_scale=sm, check=True,
+                                      precision=precision)
+        want, vmax = _f64_rows(q, pool, scales, bt, cu, qp, ranges, causal, sm)
+        assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy(), precision)
+    zero, end = t(np.zeros(len(n_q), np.int32)), t(lens.astype(np.int32))
+    out = torch.full(q.shape, 7.0, dtype=torch.bfloat16, device=DEV)
+    kv.paged_attention_prefill(q, t(cu), t(qp), pool, scales, bt, zero, end, causal=causal, out=out, max_q_per_seq=1,
+                               precision=precision)
+    rows = 32 * 4 // (4 if Hq // Hkv % 4 == 0 else 2 if Hq // Hkv % 2 == 0 else 1)  # of the one tile that is computed
+    for b, n in enumerate(n_q):
+        assert (out[int(cu[b]) + rows:int(cu[b]) + n] == 7.0).all()
+
+
+def test_ring_shard_bounds_match_torch():
+    """The shard bounds' kernel against the integer expression, negative and large lengths
+    among them; a kv_len of another dtype gives the same attention."""
+    lens = torch.tensor([0, 1, 7, 8191, 2**31 - 1, -5], dtype=torch.int32, device=DEV)
+    for R in (1, 3, 70):
+        row = 8
+        begin = torch.full((R, row), -99, dtype=torch.int32, device=DEV)
+        end = begin.clone()
+        lib = kv.N.load()
+        kv.N.check(lib.zx_ring_shard_bounds(kv.N.ptr(lens), 6, R, row, kv.N.ptr(begin), kv.N.ptr(end),
+                                            kv.N.stream_ptr(DEV)), "bounds")
+        want = lens.to(torch.int64)[None] * torch.arange(R + 1, device=DEV)[:, None] // R
+        assert torch.equal(begin[:, :6].long(), want[:-1]) and torch.equal(end[:, :6].long(), want[1:])
+        assert (begin[:, 6:] == -99).all()
+    c = _ring_case()
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    args = (c["q"].to(DEV), t(c["cu"]), t(c["qp"]), t(c["pool"]), t(c["scales"]), t(c["bt"]))
+    a = kv.ring_attention_fp8(*args, t(c["lens"]), 3)
+    b = kv.ring_attention_fp8(*args, t(c["lens"]).long(), 3)
+    assert torch.equal(a, b)

@@ -33,7 +33,7 @@ ZX_PREFILL_FINAL = 64
 ZX_HEADS_TWO_PASS = 1
 ZX_HEADS_SINGLE_PASS = 2
 ZX_NEVER = 0x7FFFFFFF
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 _P = ctypes.c_void_p
 _I64, _I32, _SZ, _INT = ctypes.c_int64, ctypes.c_int32, ctypes.c_size_t, ctypes.c_int
@@ -80,6 +80,11 @@ SIGNATURES = {
                                           _P, _I32, _I32, _I32, ctypes.c_float, _I32, _P, _P, _P, _P, _P]),
     "zx_paged_attention_ring": (_INT, [_P, _I64, _P, _P, _I32, _P, _I64, _I32, _I32, _I32, _P, _P, _I32, _P,
                                        _P, _I32, _I32, _I32, _I32, ctypes.c_float, _I32, _P, _P, _P, _P, _P]),
+    "zx_paged_attention_ring_workspace_bytes": (_SZ, [_I64, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32]),
+    "zx_paged_attention_ring_ws": (_INT, [_P, _I64, _P, _P, _I32, _P, _I64, _I32, _I32, _I32, _P, _P, _I32, _P,
+                                          _P, _I32, _I32, _I32, _I32, ctypes.c_float, _I32, _P, _P, _P, _P, _P, _SZ,
+                                          _P]),
+    "zx_ring_shard_bounds": (_INT, [_P, _I32, _I32, _I32, _P, _P, _P]),
 }
 
 _lib = None

@@ -22,6 +22,8 @@
 // At the end each row is normalised; with MERGE the step's (O, lse2) is combined with
 // the running one in o_acc / lse2 (each (row, head) belongs to one block, so no races);
 // with the bf16 flag the merged row is also written as bf16.
+#include <algorithm>
+
 #include "zx_attn_common.h"
 
 namespace zx {
@@ -50,7 +52,9 @@ struct PrefillArgs {
   int32_t *err;
   int64_t n_pages;
   int32_t n_q_heads, n_kv_heads, page_size, max_blocks, mode, causal, n_ranges, n_seqs;
-  int32_t n_qt;  // query tiles per sequence (the grid is n_qt x head groups x sequences)
+  int32_t n_qt;  // query tiles per sequence (the grid is n_qt x n_split x head groups x sequences)
+  int32_t n_split;      // blocks that share a query tile's keys; each writes a part of its own:
+  int64_t part_stride;  // rows (x heads) between the parts in o_acc / lse2
   uint32_t p_magic;
   int32_t p_shift;
   float sm_log2e;  // sm_scale * log2 e
@@ -107,7 +111,10 @@ __device__ __forceinline__ void decode16_f16(uint4 c, uint32_t (&b)[8]) {
   }
 }
 
-template <int G, int PM>
+// PARTS: the blocks share each tile's keys (a.n_split > 1).  An instantiation of its own: the
+// extra live values cost the kernel without parts 3-7% (a ring of 8 launches over 4 x 8,192
+// rows 3,081 -> 3,297 us, exact weights 2,950 -> 3,054).
+template <int G, int PM, bool PARTS>
 __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(PrefillArgs a) {
   constexpr bool EXACT = PM == PF_P_EXACT, F16 = PM == PF_P_F16;
   constexpr int D = 128;
@@ -117,8 +124,15 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
   // every second-to-last, ... (globally longest first: the shortest blocks make the tail)
   const int n_hg = a.n_q_heads / G;
   const int64_t per_rank = (int64_t)n_hg * a.n_seqs;
-  const int64_t qt_rev = (int64_t)blockIdx.x / per_rank;
+  int64_t qt_rev = (int64_t)blockIdx.x / per_rank;
   const int rem = (int)((int64_t)blockIdx.x - qt_rev * per_rank);
+  int split = 0;
+  if constexpr (PARTS) {  // parts of one tile next to each other
+    split = (int)(qt_rev % a.n_split);
+    qt_rev /= a.n_split;
+    a.o_acc += split * a.part_stride * 128;
+    a.lse2 += split * a.part_stride;
+  }
   const int hg = rem % n_hg, b = rem / n_hg;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -196,6 +210,15 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
     }
     g.ke_blk = a.causal ? (int)max((int64_t)-1, min((int64_t)g.ke, qp0 + last_row + 1)) : g.ke;
     g.s_first = (g.kb / 16) * 16;
+    if (PARTS && g.s_first < g.ke_blk) {  // this block's share of the range's steps
+      const int64_t steps = (g.ke_blk - g.s_first + PF_KEYS - 1) / PF_KEYS;
+      const int lo = g.s_first + PF_KEYS * (int)(steps * split / a.n_split);
+      const int hi = g.s_first + PF_KEYS * (int)(steps * (split + 1) / a.n_split);
+      g.kb = max(g.kb, lo);
+      g.ke = min(g.ke, hi);
+      g.ke_blk = min(g.ke_blk, hi);
+      g.s_first = lo;
+    }
     return g;
   };
   // the first range with a step at or after r (a.n_ranges if none)
@@ -1207,17 +1230,111 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
   if (e && a.err) atomicOr(a.err, e);
 }
 
+// Rows whose keys several blocks shared: out = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M)
+// over the parts (normalised fp32 rows and their log2 sums), as bf16.  A block takes a query
+// tile of a head group, as the parts' blocks did (rows no tile holds are left alone), half a
+// wave a row, 4 channels per lane; the lanes of a half hold the parts' sums.  Parts of weight
+// 0 are added too (0 x NaN: a NaN key or value makes its rows NaN whichever part held it).
+constexpr int PC_MAX = 32;  // parts
+__global__ void __launch_bounds__(256) prefill_combine_kernel(PrefillArgs a, int32_t G, int32_t qt_rows) {
+  const int n_hg = a.n_q_heads / G;
+  const int64_t per_rank = (int64_t)n_hg * a.n_seqs;
+  const int64_t qt = (int64_t)blockIdx.x / per_rank;
+  const int rem = (int)((int64_t)blockIdx.x - qt * per_rank);
+  const int hg = rem % n_hg, b = rem / n_hg;
+  const int32_t cq0 = a.cu_q[b], n_qb = a.cu_q[b + 1] - cq0;
+  const int64_t row0 = qt * qt_rows;
+  if (row0 >= n_qb) return;
+  const int n_rows = (int)min((int64_t)qt_rows, n_qb - row0) * G;  // (row, head) pairs
+  const int lane = threadIdx.x & 63, s_l = lane & 31;
+  const int S = a.n_split;
+  for (int i = threadIdx.x >> 5; i < n_rows; i += 8) {  // uniform in half a wave, where the shuffles stay
+    const int64_t row = (cq0 + row0 + i / G) * a.n_q_heads + hg * G + i % G;
+    const float ls = s_l < S ? a.lse2[s_l * a.part_stride + row] : -INFINITY;
+    float M = ls;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    const float w = M == -INFINITY || s_l >= S ? 0.0f : __builtin_amdgcn_exp2f(ls - M);
+    float L = w;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) L += __shfl_xor(L, off, 64);
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float *src = a.o_acc + row * 128 + 4 * s_l;
+    for (int s = 0; s < S; s += 4) {
+      float4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = *reinterpret_cast<const float4 *>(src + min(s + u, S - 1) * a.part_stride * 128);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float ws = __shfl(w, ((lane & 32) + s + u) & 63, 64);
+        if (s + u < S) {
+          acc.x += ws * v[u].x;
+          acc.y += ws * v[u].y;
+          acc.z += ws * v[u].z;
+          acc.w += ws * v[u].w;
+        }
+      }
+    }
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    *reinterpret_cast<uint2 *>(a.out + row * 128 + 4 * s_l) =
+        make_uint2(pack_bf16(acc.x * inv, acc.y * inv), pack_bf16(acc.z * inv, acc.w * inv));
+  }
+}
+
 }  // namespace zx
 
 using namespace zx;
 
 namespace {
+// How a call is cut into blocks.
+struct PrefillPlan {
+  int G, pm, n_split;
+  bool wide;
+};
+PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int32_t page_size, int32_t max_blocks,
+                         int32_t n_seqs, int32_t max_q_per_seq, int32_t causal, int32_t flags) {
+  PrefillPlan p;
+  const int grp = n_q_heads / n_kv_heads;
+  p.G = grp % 4 == 0 ? 4 : (grp % 2 == 0 ? 2 : 1);
+  p.pm = (flags & ZX_PREFILL_EXACT_P) ? PF_P_EXACT : ((flags & ZX_PREFILL_FAST_P) ? PF_P_BF16 : PF_P_F16);
+  const int64_t cap = (int64_t)max_blocks * page_size;  // positions a sequence can have
+  const bool rows_only = !(flags & ZX_PREFILL_MERGE);
+  // blocks of `qt` rows that hold any (sequences differ in length)
+  auto blocks = [&](int64_t qt) {
+    return std::min(ceil_div(max_q_per_seq, qt) * n_seqs, ceil_div(n_q, qt) + n_seqs) * (n_q_heads / p.G);
+  };
+  // 64 rows per wave where nothing is merged, four query heads share a KV head, there is a
+  // block per CU and contexts can be long: its blocks start and end more slowly (3 x 500-2,000
+  // rows of new sequences: 102 against 90 us; 4 x 512 rows on 8,192 cached: 329 against 346),
+  // one or two heads per KV head gained nothing (2 x 4,096: 150 against 140, 175 against 175),
+  // and the exact mode's second set of weights does not fit its registers.
+  p.wide = p.G == 4 && rows_only && p.pm != PF_P_EXACT && cap >= 4096 && blocks(PW_ROWS) >= num_cus();
+  // Few blocks: several share a tile's keys (2 x 300-700 rows on 4k-12k cached 467 -> 254 us,
+  // 256 rows on 16k 443 -> 134, 4 x 4-8 rows on 4k-8k 322 -> 59).  One round of resident blocks
+  // where that gives at least four parts a tile (256 rows on 16k: 169 us with two rounds, whose
+  // parts cost more to combine), else two, which even out sequences of different lengths (2 x
+  // 300-700: 290 us with one); at least 8 steps each (1,024 rows of a new sequence: 56 us in
+  // parts of 4 to 8 steps against 45).
+  p.n_split = 1;
+  const int64_t nb = blocks(32 * 4 / p.G), slots = 2LL * num_cus();
+  if (rows_only && !p.wide && nb > 0) {
+    const int64_t steps = (cap - (causal ? std::min<int64_t>(max_q_per_seq, cap) / 2 : 0)) / PF_KEYS;
+    const int64_t parts = slots / nb >= 4 ? slots / nb : 2 * slots / nb;
+    p.n_split = (int)std::max<int64_t>(1, std::min({parts, steps / 8, (int64_t)PC_MAX}));
+  }
+  return p;
+}
+size_t prefill_part_bytes(const PrefillPlan &p, int64_t n_q, int32_t n_q_heads) {
+  return p.n_split > 1 ? (size_t)p.n_split * n_q * n_q_heads * (128 + 1) * sizeof(float) : 0;
+}
+
 int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int32_t *q_pos0, int32_t n_q_heads,
                  const uint8_t *pool, int64_t n_pages, int32_t n_kv_heads, int32_t head_dim, int32_t page_size,
                  const float *scales, const int32_t *block_tables, int32_t max_blocks, const int32_t *kv_begin,
                  const int32_t *kv_end, int32_t n_ranges, int32_t n_seqs, int32_t max_q_per_seq, int32_t causal,
                  float sm_scale, int32_t flags, float *o_acc, float *lse2, uint16_t *out, int32_t *err,
-                 zx_stream_t stream) {
+                 void *workspace, size_t workspace_bytes, zx_stream_t stream) {
   ZX_REQUIRE(q && cu_q && q_pos0 && pool && scales && block_tables && kv_begin && kv_end,
              "paged_attention_prefill: null pointer");
   ZX_REQUIRE(n_ranges >= 1, "paged_attention: n_ranges must be positive");
@@ -1248,8 +1365,9 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
   if (n_q == 0 || max_q_per_seq == 0) return ZX_OK;
   if ((int64_t)max_blocks * page_size >= (1LL << 31))
     return fail(ZX_ERR_UNSUPPORTED, "paged_attention_prefill: sequences too long");
-  const int grp = n_q_heads / n_kv_heads;
-  const int G = grp % 4 == 0 ? 4 : (grp % 2 == 0 ? 2 : 1);
+  PrefillPlan p = prefill_plan(n_q, n_q_heads, n_kv_heads, page_size, max_blocks, n_seqs, max_q_per_seq, causal, flags);
+  if (!workspace || workspace_bytes < prefill_part_bytes(p, n_q, n_q_heads)) p.n_split = 1;  // no room for parts
+  const int G = p.G, pm = p.pm;
   PrefillArgs a;
   a.q = q;
   a.cu_q = cu_q;
@@ -1281,44 +1399,70 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
     a.p_shift = shift;
     a.p_magic = (uint32_t)(((1ULL << (31 + shift)) + page_size - 1) / page_size);
   }
-  const int pm = (flags & ZX_PREFILL_EXACT_P) ? PF_P_EXACT : ((flags & ZX_PREFILL_FAST_P) ? PF_P_BF16 : PF_P_F16);
-  // 64 rows per wave where nothing is merged, four query heads share a KV head, there is a
-  // block per CU and contexts can be long: its blocks start and end more slowly (3 x 500-2,000
-  // rows of new sequences: 102 against 90 us; 4 x 512 rows on 8,192 cached: 329 against 346),
-  // one or two heads per KV head gained nothing (2 x 4,096: 150 against 140, 175 against 175),
-  // and the exact mode's second set of weights does not fit its registers.
-  const bool wide = G == 4 && !(flags & ZX_PREFILL_MERGE) && pm != PF_P_EXACT &&
-                    (int64_t)max_blocks * page_size >= 4096 &&
-                    ceil_div(max_q_per_seq, PW_ROWS) * (n_q_heads / G) * n_seqs >= num_cus();
-  const int QT = wide ? PW_ROWS : 32 * 4 / G;
+  const int QT = p.wide ? PW_ROWS : 32 * 4 / G;
   a.n_qt = (int32_t)ceil_div(max_q_per_seq, QT);
-  const int64_t n_blocks = (int64_t)a.n_qt * (n_q_heads / G) * n_seqs;
+  const int64_t n_blocks = (int64_t)a.n_qt * p.n_split * (n_q_heads / G) * n_seqs;
   ZX_REQUIRE(n_blocks < (1LL << 31), "paged_attention_prefill: too many query tiles or sequences");
   const dim3 grid((unsigned)n_blocks);
   hipStream_t st = as_stream(stream);
-  if (wide) {
+  if (p.wide) {
     if (pm == PF_P_F16) paged_prefill_wide_kernel<PF_P_F16><<<grid, PF_THREADS, 0, st>>>(a);
     else paged_prefill_wide_kernel<PF_P_BF16><<<grid, PF_THREADS, 0, st>>>(a);
     return check_launch("paged_prefill_wide");
   }
+  a.n_split = p.n_split;
+  a.part_stride = n_q * n_q_heads;
+  if (p.n_split > 1) {  // each part writes its own normalised rows and log2 sums
+    a.o_acc = static_cast<float *>(workspace);
+    a.lse2 = a.o_acc + (int64_t)p.n_split * a.part_stride * 128;
+    a.mode = PF_MERGE | PF_INIT;
+  }
   switch (G * 4 + pm) {
-#define ZX_PF_CASE(g, m) \
-  case g * 4 + m: paged_prefill_mfma_kernel<g, m><<<grid, PF_THREADS, 0, st>>>(a); break;
-    ZX_PF_CASE(4, PF_P_F16)
-    ZX_PF_CASE(4, PF_P_BF16)
-    ZX_PF_CASE(4, PF_P_EXACT)
-    ZX_PF_CASE(2, PF_P_F16)
-    ZX_PF_CASE(2, PF_P_BF16)
-    ZX_PF_CASE(2, PF_P_EXACT)
-    ZX_PF_CASE(1, PF_P_F16)
-    ZX_PF_CASE(1, PF_P_BF16)
-    ZX_PF_CASE(1, PF_P_EXACT)
+#define ZX_PF_CASE(g, m)                                                                     \
+  case g * 4 + m:                                                                            \
+    if (p.n_split > 1) paged_prefill_mfma_kernel<g, m, true><<<grid, PF_THREADS, 0, st>>>(a); \
+    else paged_prefill_mfma_kernel<g, m, false><<<grid, PF_THREADS, 0, st>>>(a);              \
+    break;
+#define ZX_PF_CASES(g) ZX_PF_CASE(g, PF_P_F16) ZX_PF_CASE(g, PF_P_BF16) ZX_PF_CASE(g, PF_P_EXACT)
+    ZX_PF_CASES(4)
+    ZX_PF_CASES(2)
+    ZX_PF_CASES(1)
+#undef ZX_PF_CASES
 #undef ZX_PF_CASE
     default: return fail(ZX_ERR_INVALID, "paged_attention_prefill: internal dispatch");
   }
-  return check_launch("paged_prefill_mfma");
+  int rc = check_launch("paged_prefill_mfma");
+  if (rc || p.n_split == 1) return rc;
+  prefill_combine_kernel<<<(unsigned)(n_blocks / p.n_split), 256, 0, st>>>(a, G, QT);
+  return check_launch("prefill_combine");
 }
 }  // namespace
+
+extern "C" size_t zx_paged_attention_ring_workspace_bytes(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads,
+                                                          int32_t page_size, int32_t max_blocks, int32_t n_seqs,
+                                                          int32_t max_q_per_seq, int32_t causal, int32_t flags) {
+  if (n_q <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads || page_size <= 0 || max_blocks <= 0 ||
+      n_seqs <= 0 || max_q_per_seq <= 0)
+    return 0;
+  return prefill_part_bytes(
+      prefill_plan(n_q, n_q_heads, n_kv_heads, page_size, max_blocks, n_seqs, max_q_per_seq, causal, flags), n_q,
+      n_q_heads);
+}
+
+extern "C" int zx_paged_attention_ring_ws(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int32_t *q_pos0,
+                                          int32_t n_q_heads, const uint8_t *pool, int64_t n_pages, int32_t n_kv_heads,
+                                          int32_t head_dim, int32_t page_size, const float *scales,
+                                          const int32_t *block_tables, int32_t max_blocks, const int32_t *kv_begin,
+                                          const int32_t *kv_end, int32_t n_ranges, int32_t n_seqs,
+                                          int32_t max_q_per_seq, int32_t causal, float sm_scale, int32_t flags,
+                                          float *o_acc, float *lse2, uint16_t *out, int32_t *err, void *workspace,
+                                          size_t workspace_bytes, zx_stream_t stream) {
+  clear_error();
+  ZX_REQUIRE(!workspace || aligned16(workspace), "paged_attention_ring_ws: workspace must be 16-byte aligned");
+  return prefill_impl(q, n_q, cu_q, q_pos0, n_q_heads, pool, n_pages, n_kv_heads, head_dim, page_size, scales,
+                      block_tables, max_blocks, kv_begin, kv_end, n_ranges, n_seqs, max_q_per_seq, causal, sm_scale,
+                      flags, o_acc, lse2, out, err, workspace, workspace_bytes, stream);
+}
 
 extern "C" int zx_paged_attention_prefill(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int32_t *q_pos0,
                                           int32_t n_q_heads, const uint8_t *pool, int64_t n_pages, int32_t n_kv_heads,
@@ -1330,7 +1474,7 @@ extern "C" int zx_paged_attention_prefill(const uint16_t *q, int64_t n_q, const 
   clear_error();
   return prefill_impl(q, n_q, cu_q, q_pos0, n_q_heads, pool, n_pages, n_kv_heads, head_dim, page_size, scales,
                       block_tables, max_blocks, kv_begin, kv_end, 1, n_seqs, max_q_per_seq, causal, sm_scale, flags,
-                      o_acc, lse2, out, err, stream);
+                      o_acc, lse2, out, err, nullptr, 0, stream);
 }
 
 extern "C" int zx_paged_attention_ring(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int32_t *q_pos0,
@@ -1343,5 +1487,5 @@ extern "C" int zx_paged_attention_ring(const uint16_t *q, int64_t n_q, const int
   clear_error();
   return prefill_impl(q, n_q, cu_q, q_pos0, n_q_heads, pool, n_pages, n_kv_heads, head_dim, page_size, scales,
                       block_tables, max_blocks, kv_begin, kv_end, n_ranges, n_seqs, max_q_per_seq, causal, sm_scale,
-                      flags, o_acc, lse2, out, err, stream);
+                      flags, o_acc, lse2, out, err, nullptr, 0, stream);
 }

@@ -68,3 +68,30 @@ extern "C" int zx_ring_curriculum_trace(const int32_t *degrees, const int32_t *c
   }
   return ZX_OK;
 }
+
+// Shard r of a ring holds keys [floor(r n / R), floor((r + 1) n / R)) of a sequence of n.
+__global__ void ring_shards_kernel(const int32_t *__restrict__ kv_len, int32_t n_seqs, int32_t R, int64_t row_stride,
+                                   int32_t *__restrict__ kv_begin, int32_t *__restrict__ kv_end) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)R * n_seqs) return;
+  const int64_t r = i / n_seqs, b = i - r * n_seqs, n = kv_len[b];
+  auto bound = [&](int64_t k) {  // floor, for a negative length too
+    const int64_t q = n * k / R;
+    return (int32_t)(q - (n * k - q * R < 0));
+  };
+  kv_begin[r * row_stride + b] = bound(r);
+  kv_end[r * row_stride + b] = bound(r + 1);
+}
+
+extern "C" int zx_ring_shard_bounds(const int32_t *kv_len, int32_t n_seqs, int32_t degree, int32_t row_stride,
+                                    int32_t *kv_begin, int32_t *kv_end, zx_stream_t stream) {
+  clear_error();
+  ZX_REQUIRE(n_seqs >= 0 && degree >= 1 && row_stride >= n_seqs, "ring_shard_bounds: bad sizes");
+  if (n_seqs == 0) return ZX_OK;
+  ZX_REQUIRE(kv_len && kv_begin && kv_end, "ring_shard_bounds: null pointer");
+  const int64_t blocks = ceil_div((int64_t)degree * n_seqs, 256);
+  ZX_REQUIRE(blocks < (1LL << 31), "ring_shard_bounds: too many shards");
+  ring_shards_kernel<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(kv_len, n_seqs, degree, row_stride, kv_begin,
+                                                                      kv_end);
+  return check_launch("ring_shards");
+}

@@ -413,6 +413,15 @@ def _precision_flag(precision: str) -> int:
     raise ValueError(f"precision must be one of {PRECISIONS}, got {precision!r}")
 
 
+def _parts_workspace(q: torch.Tensor, Hkv: int, P: int, block_tables: torch.Tensor, B: int, max_q_per_seq: int,
+                     causal: bool, flags: int):
+    """Workspace (and its bytes) of a call that the library cuts along the keys; (None, 0)
+    when it does not."""
+    nb = N.load().zx_paged_attention_ring_workspace_bytes(q.shape[0], q.shape[1], Hkv, P, block_tables.shape[1], B,
+                                                          int(max_q_per_seq), int(bool(causal)), flags)
+    return (_workspace(nb, q.device), nb) if nb else (None, 0)
+
+
 def paged_attention_prefill(q: torch.Tensor, cu_q: torch.Tensor, q_pos0: torch.Tensor, pool_layer: torch.Tensor,
                             scales_layer: torch.Tensor, block_tables: torch.Tensor, kv_begin: torch.Tensor,
                             kv_end: torch.Tensor, causal: bool = True, sm_scale: float | None = None,
@@ -491,11 +500,19 @@ def paged_attention_prefill(q: torch.Tensor, cu_q: torch.Tensor, q_pos0: torch.T
         err = _err_word_if(check, dev)
     elif err.dtype != torch.int32 or err.numel() < 1 or err.device != dev:
         raise ValueError("err must be an int32 tensor on q's device")
-    N.check(N.load().zx_paged_attention_prefill(
-        N.ptr(q), n_q, N.ptr(cu_q), N.ptr(q_pos0), Hq, N.ptr(pool_layer), n_pages, Hkv, D, P, N.ptr(scales_layer),
-        N.ptr(block_tables), block_tables.shape[1], N.ptr(kv_begin), N.ptr(kv_end), B, int(max_q_per_seq),
-        int(bool(causal)), sm, flags, N.ptr(o_acc), N.ptr(lse2), N.ptr(out if write_bf16 else None), N.ptr(err),
-        N.stream_ptr(dev)), "paged_attention_prefill")
+    lib = N.load()
+    args = (N.ptr(q), n_q, N.ptr(cu_q), N.ptr(q_pos0), Hq, N.ptr(pool_layer), n_pages, Hkv, D, P, N.ptr(scales_layer),
+            N.ptr(block_tables), block_tables.shape[1], N.ptr(kv_begin), N.ptr(kv_end))
+    if o_acc is None:
+        ws, nb = _parts_workspace(q, Hkv, P, block_tables, B, max_q_per_seq, causal, flags)
+        rc = lib.zx_paged_attention_ring_ws(*args, 1, B, int(max_q_per_seq), int(bool(causal)), sm, flags, None, None,
+                                            N.ptr(out if write_bf16 else None), N.ptr(err), N.ptr(ws), nb,
+                                            N.stream_ptr(dev))
+    else:
+        rc = lib.zx_paged_attention_prefill(*args, B, int(max_q_per_seq), int(bool(causal)), sm, flags, N.ptr(o_acc),
+                                            N.ptr(lse2), N.ptr(out if write_bf16 else None), N.ptr(err),
+                                            N.stream_ptr(dev))
+    N.check(rc, "paged_attention_prefill")
     if check:
         _raise_kernel_error(err, "paged_attention_prefill")
     return out if write_bf16 else None
@@ -542,11 +559,12 @@ def paged_attention_ring(q: torch.Tensor, cu_q: torch.Tensor, q_pos0: torch.Tens
     sm = float(sm_scale) if sm_scale is not None else 1.0 / float(D) ** 0.5
     if err is None:
         err = _err_word_if(check, q.device)
-    N.check(N.load().zx_paged_attention_ring(
+    flags = N.ZX_PREFILL_BF16 | p_flag
+    ws, nb = _parts_workspace(q, Hkv, P, block_tables, B, max_q_per_seq, causal, flags)
+    N.check(N.load().zx_paged_attention_ring_ws(
         N.ptr(q), n_q, N.ptr(cu_q), N.ptr(q_pos0), Hq, N.ptr(pool_layer), n_pages, Hkv, D, P, N.ptr(scales_layer),
         N.ptr(block_tables), block_tables.shape[1], N.ptr(kv_begin), N.ptr(kv_end), kv_begin.shape[0], B,
-        int(max_q_per_seq), int(bool(causal)), sm, N.ZX_PREFILL_BF16 | p_flag, None,
-        None, N.ptr(out), N.ptr(err),
+        int(max_q_per_seq), int(bool(causal)), sm, flags, None, None, N.ptr(out), N.ptr(err), N.ptr(ws), nb,
         N.stream_ptr(q.device)), "paged_attention_ring")
     if check:
         _raise_kernel_error(err, "paged_attention_ring")
@@ -581,21 +599,29 @@ def ring_attention_fp8(q: torch.Tensor, cu_q: torch.Tensor, q_pos0: torch.Tensor
         mq = int((cu_q[1:] - cu_q[:-1]).max().item()) if cu_q.numel() > 1 else 0
     else:
         mq = int(max_q_per_seq)
-    # Shard r covers keys [kv_len * r // R, kv_len * (r + 1) // R): all bounds in one go,
-    # so the loop below only launches the ring steps (rows padded to 16 bytes, the
-    # alignment every pointer of the C ABI needs).
+    # Shard r covers keys [kv_len * r // R, kv_len * (r + 1) // R): all bounds in one go (one
+    # small kernel; any other kind of kv_len as torch computes it).  Each ring step takes a
+    # row of its own, padded to 16 bytes (the alignment the wrappers ask for); one launch
+    # takes rows without gaps.
     B = kv_len.numel()
-    steps = torch.arange(ring_degree + 1, dtype=torch.int64, device=kv_len.device)
-    bounds = torch.empty((ring_degree + 1, (B + 3) // 4 * 4), dtype=torch.int32, device=kv_len.device)
-    bounds[:, :B] = kv_len.to(torch.int64)[None, :] * steps[:, None] // ring_degree
+    R = ring_degree
+    row = B if single_launch else (B + 3) // 4 * 4
+    both = torch.empty((2, (R * row + 3) // 4 * 4), dtype=torch.int32, device=kv_len.device)
+    begin, end = (t[:R * row].view(R, row) for t in both)
+    if kv_len.dtype == torch.int32 and kv_len.dim() == 1 and kv_len.is_cuda and kv_len.is_contiguous():
+        N.check(N.load().zx_ring_shard_bounds(N.ptr(kv_len), B, R, row, N.ptr(begin), N.ptr(end),
+                                              N.stream_ptr(kv_len.device)), "ring_attention_fp8")
+    else:
+        steps = torch.arange(R + 1, dtype=torch.int64, device=kv_len.device)
+        bounds = kv_len.to(torch.int64)[None, :] * steps[:, None] // R
+        begin[:, :B], end[:, :B] = bounds[:-1], bounds[1:]
     if err is None:
         err = _err_word_if(check, q.device)
     elif err.dtype != torch.int32 or err.numel() < 1 or err.device != q.device:
         raise ValueError("err must be an int32 tensor on q's device")
     if single_launch:
-        out = paged_attention_ring(q, cu_q, q_pos0, pool_layer, scales_layer, block_tables,
-                                   bounds[:-1, :B].contiguous(), bounds[1:, :B].contiguous(), causal=causal,
-                                   sm_scale=sm_scale, max_q_per_seq=mq, err=err, precision=precision)
+        out = paged_attention_ring(q, cu_q, q_pos0, pool_layer, scales_layer, block_tables, begin, end,
+                                   causal=causal, sm_scale=sm_scale, max_q_per_seq=mq, err=err, precision=precision)
         if check:
             _raise_kernel_error(err, "ring_attention_fp8")
         return out
@@ -603,8 +629,7 @@ def ring_attention_fp8(q: torch.Tensor, cu_q: torch.Tensor, q_pos0: torch.Tensor
     lse2 = torch.empty((n_q, Hq), dtype=torch.float32, device=q.device)
     out = torch.empty_like(q)
     for r in range(ring_degree):
-        paged_attention_prefill(q, cu_q, q_pos0, pool_layer, scales_layer, block_tables, bounds[r, :B],
-                                bounds[r + 1, :B],
+        paged_attention_prefill(q, cu_q, q_pos0, pool_layer, scales_layer, block_tables, begin[r, :B], end[r, :B],
                                 causal=causal, sm_scale=sm_scale, o_acc=o_acc, lse2=lse2, first=r == 0, out=out,
                                 write_bf16=causal or r == ring_degree - 1, max_q_per_seq=mq, err=err,
                                 precision=precision, last=r == ring_degree - 1, final=causal)
