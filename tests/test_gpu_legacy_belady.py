@@ -92,6 +92,31 @@ def test_int8_legacy_every_input_below_amax(dev, dt):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f32"])
+@pytest.mark.parametrize("n_slabs,rounds,extra", [(1, 3, 5), (1, "slots", 0), (1, "slots", 8), (5, "slots", 0), (3000, 0, 24)])
+def test_int8_legacy_maximum_per_block(dev, dt, n_slabs, rounds, extra):
+    """A maximum per block against atomics on one word (a workspace of the least size): the
+    same bytes, with each slab's peak where only the last block sees it; one round per
+    block, a vector more than that, and more slabs than block slots.  No tolerance."""
+    w = 4 if dt == "f32" else 8
+    slots = torch.cuda.get_device_properties(dev).multi_processor_count * 8 // n_slabs
+    n = (slots if rounds == "slots" else rounds) * 1024 * w + extra
+    x = torch.rand((n_slabs, n), device=dev, generator=torch.Generator(dev).manual_seed(n)).to(DTYPES[dt])
+    x[:, -1] = torch.arange(n_slabs, device=dev).to(x.dtype) + 2
+    q, s = kv.int8_legacy_quant_slabs(x)
+    q2, s2 = torch.empty_like(q), torch.empty_like(s)
+    ws = torch.empty((n_slabs * 4 + 255) // 256 * 256, dtype=torch.uint8, device=dev)
+    N.check(N.load().zx_int8_legacy_quant_slabs(N.ptr(x), kv._DT[x.dtype], n_slabs, n, N.ptr(q2), N.ptr(s2), N.ptr(ws),
+                                                ws.numel(), N.stream_ptr(dev)), "int8_legacy_quant_slabs")
+    assert torch.equal(q, q2) and raw(s).tobytes() == raw(s2).tobytes()
+    want_q, want_s = O.int8_legacy_quant(raw(x[-1]), dt)  # the whole of the last slab
+    np.testing.assert_array_equal(q[-1].cpu().numpy(), want_q)
+    assert np.float32(s[-1].float().item()).tobytes() == np.float32(want_s).tobytes()
+    if n_slabs == 1:
+        q1, s1 = kv.int8_legacy_quant(x[0])
+        assert torch.equal(q1, q[0]) and torch.equal(s1, s[0])
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
 def test_int8_legacy_unaligned_view(dev, dt):
     """A view starting one element in (not 16-byte aligned) takes the element-by-element
     path; results equal the oracle's."""

@@ -76,7 +76,7 @@ def int8_legacy_quant(x: torch.Tensor):
     N.require_device(x, "x")
     q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     scale = torch.empty((), dtype=x.dtype, device=x.device)
-    ws = _workspace(256, x.device)
+    ws = _workspace(N.load().zx_int8_legacy_quant_slabs_workspace_bytes(1), x.device)
     N.check(N.load().zx_int8_legacy_quant(N.ptr(x), _DT[x.dtype], x.numel(), N.ptr(q), N.ptr(scale),
                                           N.ptr(ws), ws.numel(), N.stream_ptr(x.device)),
             "quantize_to_fp8_storage")
