@@ -265,6 +265,39 @@ def test_kv_quant_append_static_scales_decode_positions(dev):
     np.testing.assert_array_equal(pool_d.cpu().numpy(), wpool)
 
 
+@pytest.mark.parametrize("H,D,P,n_seqs,total", [
+    (2, 64, 16, 1, 16383), (2, 64, 16, 7, 16384), (2, 64, 16, 64, 16385),  # 1,024 blocks on 256 CUs, and more
+    (1, 64, 5, 130, 300), (2, 256, 7, 33, 129), (8, 128, 16, 2, 3),  # rows per wave, whole rows, a ragged tile
+])
+@pytest.mark.parametrize("static", [True, False])
+def test_kv_quant_append_finds_pages(dev, H, D, P, n_seqs, total, static):
+    """Token positions and error bits whichever kernel searches them: empty sequences, one
+    whose table is too short and one with a page id out of range, bytes equal to the oracle's."""
+    L = 2
+    g = torch.Generator().manual_seed(total)
+    cuts = torch.sort(torch.randint(0, total + 1, (n_seqs - 1,), generator=g)).values.tolist()
+    edges = [0] + cuts + [total]
+    lens = [b - a for a, b in zip(edges, edges[1:])]
+    x, cu, bt, n_pages, sp = make_append_case(L, H, D, P, lens, seed=total, start=[3 * i % 11 for i in range(n_seqs)])
+    longest = int(np.argmax(lens))
+    if n_seqs > 2:
+        sp[longest] = bt.shape[1] * P - lens[longest] // 2  # half of its tokens lie past the table
+        bt[longest, -1] = n_pages + 2
+    scales = torch.rand((L, 2, H), dtype=torch.float32, generator=g) + 1
+    pool = torch.zeros((L, n_pages, 2, H, P, D), dtype=torch.uint8)
+    wpool = pool.numpy().copy()
+    wsc, werr = O.kv_quant_append(bits16(x), cu.numpy(), sp.numpy(), bt.numpy(), wpool, P,
+                                  scales=scales.numpy() if static else None)
+    assert werr == (3 if n_seqs > 2 else 0)
+    pool_d, err = pool.to(dev), torch.zeros(1, dtype=torch.int32, device=dev)
+    sc = kv.kv_quant_append(x.to(dev), cu.to(dev), bt.to(dev), pool_d, scales=scales.to(dev) if static else None,
+                            start_pos=sp.to(dev), static_scales=static, err=err, two_pass=not static)
+    assert int(err.item()) == werr
+    np.testing.assert_array_equal(sc.cpu().numpy().view(np.uint32),
+                                  scales.numpy().view(np.uint32) if static else wsc.view(np.uint32))
+    np.testing.assert_array_equal(pool_d.cpu().numpy(), wpool)
+
+
 def test_kv_quant_append_rejects_bad_page_ids(dev):
     L, H, D, P = 1, 2, 64, 16
     x, cu, bt, n_pages, _ = make_append_case(L, H, D, P, [20, 5], seed=3)
