@@ -122,8 +122,8 @@ size_t zx_fp8_quant_heads_workspace_bytes(int64_t n_outer, int64_t n_batch, int6
  * workgroups than the device holds (n_batch * ceil(run / 46080) > compute units), an input
  * below 256 MiB without ZX_HEADS_SINGLE_PASS (the Infinity Cache serves the second read
  * there, making two passes faster), or ZX_HEADS_TWO_PASS take two passes (same results).
- * workspace: zx_fp8_quant_heads_workspace_bytes() device bytes (unused with two passes,
- * may then be NULL). */
+ * workspace: zx_fp8_quant_heads_workspace_bytes() device bytes (two passes take less, or
+ * NULL, too: with it they need two launches fewer). */
 int zx_fp8_quant_heads(const uint16_t *x, int64_t n_outer, int64_t n_batch, int64_t n_heads,
                        int64_t run, uint8_t *codes, float *scales, int32_t flags, int32_t *err,
                        void *workspace, size_t workspace_bytes, zx_stream_t stream);

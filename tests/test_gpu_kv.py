@@ -159,6 +159,38 @@ def test_fp8_heads_special_slabs(dev):
     assert_bf16_equal(bits16(kv.fp8_dequant_heads(codes, scales)), O.fp8_dequant_heads(wc, ws))
 
 
+@pytest.mark.parametrize("n_outer,B,H,run", [
+    (1, 1, 1, 16), (3, 2, 5, 16 * 1024), (2, 3, 2, 16 * 1024 + 16),  # one chunk, one and a bit
+    (1, 2, 2, 128 * 16 * 1024), (1, 1, 3, 256 * 16 * 1024 + 16),  # the most stored maxima, and one more
+])
+def test_fp8_heads_stored_maxima(dev, n_outer, B, H, run):
+    """Two passes with each block's maximum stored, in both workspace sizes: every slab's
+    maximum in another chunk, one slab of zeros, one with a NaN and one with an infinity."""
+    lib = kv.N.load()
+    x = torch.randn((n_outer, B, H, run), generator=torch.Generator().manual_seed(run)).to(torch.bfloat16)
+    flat = x.permute(0, 2, 1, 3).reshape(n_outer * H, B * run).clone()
+    n = B * run
+    for i in range(n_outer * H):
+        flat[i, (i * 7919 + n - 1) % n] = -50.0 - i
+    if n_outer * H > 3:
+        flat[1] = 0
+        flat[2, n // 2] = float("nan")
+        flat[3, n - 1] = float("inf")
+    x = flat.view(n_outer, H, B, run).permute(0, 2, 1, 3).contiguous()
+    wc, want = O.fp8_quant_heads(bits16(x))
+    xd = x.to(dev)
+    for ws_bytes in (lib.zx_fp8_quant_heads_workspace_bytes(n_outer, B, H, run), 0):
+        codes = torch.empty(x.shape, dtype=torch.uint8, device=dev)
+        scales = torch.full((n_outer, H), -1.0, device=dev)
+        ws = torch.full((max(ws_bytes, 1),), 255, dtype=torch.uint8, device=dev)
+        kv.N.check(lib.zx_fp8_quant_heads(kv.N.ptr(xd), n_outer, B, H, run, kv.N.ptr(codes), kv.N.ptr(scales),
+                                          kv.N.ZX_HEADS_TWO_PASS, None, kv.N.ptr(ws) if ws_bytes else None, ws_bytes,
+                                          kv.N.stream_ptr(xd.device)), "fp8_quant_heads")
+        np.testing.assert_array_equal(scales.cpu().numpy().view(np.uint32), want.view(np.uint32))
+        np.testing.assert_array_equal(codes.cpu().numpy(), wc)
+
+
+
 def make_append_case(L, H, D, P, lens, seed, extra_pages=7, start=None):
     g = torch.Generator().manual_seed(seed)
     B = len(lens)

@@ -169,12 +169,12 @@ def fp8_quant_heads(x: torch.Tensor, two_pass: bool = False, check: bool = False
     lib = N.load()
     if two_pass and single_pass:
         raise ValueError("fp8_quant_heads: two_pass and single_pass are exclusive")
-    ws = None if two_pass else _workspace(lib.zx_fp8_quant_heads_workspace_bytes(O, B, H, R), x.device)
+    ws = _workspace(lib.zx_fp8_quant_heads_workspace_bytes(O, B, H, R), x.device)
     err = _err_word_if(check, x.device)
     flags = N.ZX_HEADS_TWO_PASS if two_pass else (N.ZX_HEADS_SINGLE_PASS if single_pass else 0)
     N.check(lib.zx_fp8_quant_heads(N.ptr(x), O, B, H, R, N.ptr(codes), N.ptr(scales),
-                                   flags, N.ptr(err), N.ptr(ws),
-                                   0 if ws is None else ws.numel(), N.stream_ptr(x.device)), "fp8_quant_heads")
+                                   flags, N.ptr(err), N.ptr(ws), ws.numel(), N.stream_ptr(x.device)),
+            "fp8_quant_heads")
     if check:
         _raise_kernel_error(err, "fp8_quant_heads")
     return codes, scales
