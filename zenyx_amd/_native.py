@@ -132,7 +132,7 @@ def check(rc: int, what: str) -> None:
 
 
 def require_device(t: torch.Tensor, name: str) -> None:
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be a HIP device tensor, got {t.device}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
@@ -141,16 +141,24 @@ def require_device(t: torch.Tensor, name: str) -> None:
 
 
 def ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream_ptr(device: torch.device | None = None):
     """The current torch stream of `device` as a hipStream_t."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if device is not None and device.index is not None:  # a tensor's device: no Stream object is made
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
+
+
+def need_gpu() -> None:
+    """Raises unless a HIP device is visible (not asked again of an initialised torch) and the
+    library is built.  Every wrapper begins with it."""
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
+        raise RuntimeError("zenyx_amd needs a HIP device (MI355X); none is visible")
+    load()
 
 
 def ensure_gpu() -> torch.device:
-    if not torch.cuda.is_available():
-        raise RuntimeError("zenyx_amd needs a HIP device (MI355X); none is visible")
-    load()
+    need_gpu()
     return torch.device("cuda", torch.cuda.current_device())

@@ -66,7 +66,7 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
 
 def int8_legacy_quant(x: torch.Tensor):
     """zenyx/streaming/precision.py:8-12 on the GPU: (q int8, 0-dim scale in x.dtype)."""
-    N.ensure_gpu()
+    N.need_gpu()
     if x.dtype not in _DT:
         raise TypeError(f"quantize_to_fp8_storage: unsupported dtype {x.dtype}")
     if x.numel() == 0:
@@ -85,7 +85,7 @@ def int8_legacy_quant(x: torch.Tensor):
 
 def int8_legacy_dequant(q: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
     """zenyx/streaming/precision.py:15-16 on the GPU."""
-    N.ensure_gpu()
+    N.need_gpu()
     if q.dtype != torch.int8:
         q = q.to(torch.int8)
     q = q.contiguous()
@@ -104,7 +104,7 @@ def int8_legacy_quant_slabs(x: torch.Tensor):
     """precision.py:8-12 applied to every slab ``x[i]`` of ``x [n_slabs, ...]`` in one launch:
     (q int8 like x, scales ``[n_slabs]`` in x.dtype), bit-identical to
     ``int8_legacy_quant(x[i])`` for every i."""
-    N.ensure_gpu()
+    N.need_gpu()
     if x.dtype not in _DT:
         raise TypeError(f"quantize_to_fp8_storage: unsupported dtype {x.dtype}")
     if x.dim() < 1 or x.shape[0] == 0 or x[0].numel() == 0:
@@ -123,7 +123,7 @@ def int8_legacy_quant_slabs(x: torch.Tensor):
 
 def int8_legacy_dequant_slabs(q: torch.Tensor, scales: torch.Tensor) -> torch.Tensor:
     """precision.py:15-16 applied to every slab: bf16 ``y[i] = (q[i].float() * scales[i]).to(bf16)``."""
-    N.ensure_gpu()
+    N.need_gpu()
     if q.dtype != torch.int8 or q.dim() < 1:
         raise ValueError("q must be int8 [n_slabs, ...]")
     if scales.dtype not in _DT or scales.shape != (q.shape[0],):
@@ -159,7 +159,7 @@ def fp8_quant_heads(x: torch.Tensor, two_pass: bool = False, check: bool = False
     are read once (the single-pass kernel), smaller ones in two passes (the second read
     comes from the Infinity Cache); ``two_pass`` / ``single_pass`` force either path (same
     results)."""
-    N.ensure_gpu()
+    N.need_gpu()
     if x.dtype != torch.bfloat16 or x.dim() != 4:
         raise ValueError("fp8_quant_heads: x must be bf16 [n_outer, n_batch, n_heads, run]")
     N.require_device(x, "x")
@@ -181,7 +181,7 @@ def fp8_quant_heads(x: torch.Tensor, two_pass: bool = False, check: bool = False
 
 
 def fp8_dequant_heads(codes: torch.Tensor, scales: torch.Tensor) -> torch.Tensor:
-    N.ensure_gpu()
+    N.need_gpu()
     if codes.dtype != torch.uint8 or codes.dim() != 4:
         raise ValueError("fp8_dequant_heads: codes must be uint8 [n_outer, n_batch, n_heads, run]")
     O, B, H, R = codes.shape
@@ -197,7 +197,7 @@ def fp8_dequant_heads(codes: torch.Tensor, scales: torch.Tensor) -> torch.Tensor
 
 def fp8_encode_f32(v: torch.Tensor) -> torch.Tensor:
     """Already-scaled fp32 values -> e4m3fn codes (uint8), nearest-even, overflow -> NaN."""
-    N.ensure_gpu()
+    N.need_gpu()
     if v.dtype != torch.float32:
         raise ValueError("fp8_encode_f32: v must be float32")
     v = v.contiguous()
@@ -222,7 +222,7 @@ def _layers(x: torch.Tensor):
 
 def kv_scales(x: torch.Tensor) -> torch.Tensor:
     """Per-(layer, kv, head) FP8 scales of a token-major batch -> ``[L, 2, H]`` fp32."""
-    N.ensure_gpu()
+    N.need_gpu()
     x = _layers(x)
     N.require_device(x, "x")
     L, T, _, H, D = x.shape
@@ -249,7 +249,7 @@ def kv_quant_append(x: torch.Tensor, cu_seqlens: torch.Tensor, block_tables: tor
     scales take one cooperative pass or two passes, whichever the library expects to be
     faster for the call's size; ``two_pass`` / ``single_pass`` force either (same results).
     """
-    N.ensure_gpu()
+    N.need_gpu()
     x = _layers(x)
     if pool.dim() == 5:
         pool = pool.unsqueeze(0)
@@ -300,7 +300,7 @@ def _aligned_scales(scales_layer: torch.Tensor) -> torch.Tensor:
     """One layer's ``[2, H]`` scales as the C ABI takes every pointer (contiguous, 16-byte
     aligned).  A layer of a ``[L, 2, H]`` tensor starts 8 H bytes after the previous one,
     so with H odd every other layer is not aligned: such a slice is copied (2 H floats)."""
-    if scales_layer.device.type != "cuda" or (scales_layer.is_contiguous() and scales_layer.data_ptr() % 16 == 0):
+    if not scales_layer.is_cuda or (scales_layer.is_contiguous() and scales_layer.data_ptr() % 16 == 0):
         return scales_layer
     return scales_layer.clone(memory_format=torch.contiguous_format)
 
@@ -311,7 +311,7 @@ def kv_gather_dequant(pool_layer: torch.Tensor, scales_layer: torch.Tensor, bloc
     """Paged gather + dequant of one layer: pool ``[n_pages, 2, H, P, D]`` uint8, scales
     ``[2, H]`` fp32 -> (k, v), each bf16 ``[B, H, out_len, D]``; positions at or beyond
     ``seq_lens[b]`` are zeros."""
-    N.ensure_gpu()
+    N.need_gpu()
     if pool_layer.dim() != 5 or pool_layer.dtype != torch.uint8 or pool_layer.shape[1] != 2:
         raise ValueError("pool_layer must be uint8 [n_pages, 2, H, P, D]")
     n_pages, _, H, P, D = pool_layer.shape
@@ -355,7 +355,7 @@ def paged_attention_decode(q: torch.Tensor, pool_layer: torch.Tensor, scales_lay
     ``[B, Hq, D]`` bf16 = softmax(sm_scale * q K^T) V over positions < seq_lens[b], with
     K, V = decoded codes times their head's scale (query head i reads kv head
     i // (Hq / Hkv)).  ``sm_scale`` defaults to 1/sqrt(D)."""
-    N.ensure_gpu()
+    N.need_gpu()
     if pool_layer.dim() != 5 or pool_layer.dtype != torch.uint8 or pool_layer.shape[1] != 2:
         raise ValueError("pool_layer must be uint8 [n_pages, 2, Hkv, P, D]")
     n_pages, _, Hkv, P, D = pool_layer.shape
@@ -643,7 +643,7 @@ def belady_argmax(keys: torch.Tensor, resident: torch.Tensor | None = None,
     """belady.py:39-51 over slots: device int64 ``[slot, key]`` ({-1, -1} if none).
     ``resident`` (uint8, default: every slot) selects the candidates; ``rank`` (int64,
     default: the slot index) breaks ties, smallest first."""
-    N.ensure_gpu()
+    N.need_gpu()
     if keys.dtype != torch.int64:
         raise ValueError("keys must be int64")
     N.require_device(keys, "keys")
@@ -665,7 +665,7 @@ def belady_argmax(keys: torch.Tensor, resident: torch.Tensor | None = None,
 
 def next_use(trace: torch.Tensor, n_pages: int, check: bool = False):
     """Next/previous use of every position of an int32 page trace (ZX_NEVER / -1)."""
-    N.ensure_gpu()
+    N.need_gpu()
     if trace.dtype != torch.int32 or trace.dim() != 1:
         raise ValueError("trace must be a 1-D int32 tensor")
     N.require_device(trace, "trace")
@@ -692,7 +692,7 @@ class BeladyTraceSim:
 
     def __init__(self, trace: torch.Tensor, n_pages: int, capacity: int, evict_cap: int | None = None,
                  record_misses: bool = False):
-        N.ensure_gpu()
+        N.need_gpu()
         if trace.dtype != torch.int32 or trace.dim() != 1:
             raise ValueError("trace must be a 1-D int32 device tensor")
         if capacity < 1:
