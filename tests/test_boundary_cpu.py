@@ -5,6 +5,8 @@ sequence, tiering sizes, reference timeline) matches the oracle and closed forms
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -67,6 +69,25 @@ def test_workspace_queries_are_host_only():
     assert lib.zx_kv_quant_append_workspace_bytes(32, 74902, 8, 128) >= 74902 * 8
     assert lib.zx_belady_simulate_workspace_bytes(20_971_520, 1_310_720) >= (20_971_520 + 1_310_720) // 8
     assert lib.zx_belady_argmax_workspace_bytes(1000) >= 16
+
+
+def test_decode_workspace_of_unsupported_head_dims():
+    """The wrapper asks for the size before the call is checked: for a head_dim no kernel takes
+    the answer is 0, and the call itself is refused.  In a process of its own: a division by
+    zero here would end it."""
+    code = """
+import ctypes
+from zenyx_amd import _native as N
+lib, p = N.load(), ctypes.c_void_p(16)
+for d in (-8, 0, 1, 8, 15, 96, 512, 4096, 8192, 1 << 20):
+    assert lib.zx_paged_attention_decode_workspace_bytes(1, 8, 8, d, 4, 16) == 0, d
+    rc = lib.zx_paged_attention_decode(p, 8, p, 4, 8, d, 16, p, p, 4, p, 1, 0.1, p, None, p, 1 << 20, None)
+    assert rc == N.ZX_ERR_UNSUPPORTED and b"head_dim" in lib.zx_last_error(), (d, rc)
+for d in (64, 128, 256):
+    assert lib.zx_paged_attention_decode_workspace_bytes(1, 8, 8, d, 4, 16) > 0
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stderr[-2000:])
 
 
 @pytest.mark.parametrize("L,R,S", [(1, 1, 5), (3, 8, 4), (2, 4, 7)])

@@ -867,6 +867,9 @@ static int32_t att_group(int32_t grp, bool mfma) {
   return g;
 }
 
+// The head_dims the kernels are built for; the plan below holds for these only.
+static bool att_dim_ok(int32_t head_dim) { return head_dim == 64 || head_dim == 128 || head_dim == 256; }
+
 // Blocks per group of query heads, and how the sequences are dealt to them.
 struct AttnPlan {
   bool mfma, whole;
@@ -896,7 +899,7 @@ static AttnPlan att_plan(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads, 
 
 extern "C" size_t zx_paged_attention_decode_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads,
                                                             int32_t head_dim, int32_t max_blocks, int32_t page_size) {
-  if (n_seqs <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads || head_dim <= 0 ||
+  if (n_seqs <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads || !att_dim_ok(head_dim) ||
       max_blocks <= 0 || page_size <= 0)
     return 0;
   const AttnPlan p = att_plan(n_seqs, n_q_heads, n_kv_heads, head_dim, max_blocks, page_size);
@@ -945,7 +948,7 @@ extern "C" int zx_paged_attention_decode(const uint16_t *q, int32_t n_q_heads, c
   ZX_REQUIRE(n_q_heads > 0 && n_kv_heads > 0 && n_pages > 0 && page_size > 0 && max_blocks > 0 && n_seqs > 0,
              "paged_attention_decode: sizes must be positive");
   ZX_REQUIRE(n_q_heads % n_kv_heads == 0, "paged_attention_decode: n_q_heads must be a multiple of n_kv_heads");
-  if (!(head_dim == 64 || head_dim == 128 || head_dim == 256))
+  if (!att_dim_ok(head_dim))
     return fail(ZX_ERR_UNSUPPORTED, "paged_attention_decode: head_dim %d not in {64, 128, 256}", head_dim);
   if (n_seqs > 65535) return fail(ZX_ERR_UNSUPPORTED, "paged_attention_decode: more than 65535 sequences");
   const size_t need =
