@@ -193,3 +193,21 @@ def test_attention_precision_names():
         kv.ring_attention_fp8(t, t, t, t, t, t, t, ring_degree=1, precision="fp8")
     with pytest.raises(ValueError, match="precision"):
         kv.paged_attention_prefill(t, t, t, t, t, t, t, t, precision="half")
+
+
+def test_stream_of_every_way_to_name_a_device(monkeypatch):
+    """A torch.device with an index takes the short way; a text, a number, no index and None
+    are left to torch, as it names devices."""
+    import torch
+
+    from zenyx_amd import _native as N
+
+    class Stream:
+        cuda_stream = 77
+
+    asked = []
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: asked.append(d) or Stream())
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 1000 + i, raising=False)
+    assert N.stream_ptr(torch.device("cuda", 3)) == 1003 and asked == []
+    others = ["cuda", "cuda:0", 1, torch.device("cuda"), None]
+    assert [N.stream_ptr(d) for d in others] == [77] * 5 and asked == others

@@ -144,9 +144,9 @@ def ptr(t: torch.Tensor | None):
     return None if t is None else t.data_ptr()
 
 
-def stream_ptr(device: torch.device | None = None):
-    """The current torch stream of `device` as a hipStream_t."""
-    if device is not None and device.index is not None:  # a tensor's device: no Stream object is made
+def stream_ptr(device: torch.device | str | int | None = None):
+    """The current torch stream of `device` (as torch names one) as a hipStream_t."""
+    if isinstance(device, torch.device) and device.index is not None:  # a tensor's device: no Stream object is made
         return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
