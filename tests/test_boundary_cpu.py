@@ -211,3 +211,26 @@ def test_stream_of_every_way_to_name_a_device(monkeypatch):
     assert N.stream_ptr(torch.device("cuda", 3)) == 1003 and asked == []
     others = ["cuda", "cuda:0", 1, torch.device("cuda"), None]
     assert [N.stream_ptr(d) for d in others] == [77] * 5 and asked == others
+
+
+@pytest.mark.parametrize("single_launch", [True, False])
+@pytest.mark.parametrize("form", ["int32", "int64", "row", "strided", "row_int64"])
+def test_ring_shard_bounds_of_every_kv_len(monkeypatch, form, single_launch):
+    """ring_attention_fp8 hands shard r the keys [floor(n r / R), floor(n (r + 1) / R)) whatever
+    the dtype, strides or leading dimensions of 1 of kv_len (on the CPU: by torch)."""
+    import torch
+
+    from zenyx_amd import kv
+
+    lens, R = torch.tensor([0, 5, 8191, 2**31 - 1, 17], dtype=torch.int32), 3
+    kv_len = {"int32": lens, "int64": lens.long(), "row": lens[None], "row_int64": lens.long()[None],
+              "strided": torch.stack([lens, lens], 1)[:, 0]}[form]
+    got = []
+    monkeypatch.setattr(kv, "paged_attention_ring", lambda q, cu, qp, pool, sc, bt, kb, ke, **_: got.extend(
+        zip(kb.tolist(), ke.tolist())))
+    monkeypatch.setattr(kv, "paged_attention_prefill", lambda q, cu, qp, pool, sc, bt, kb, ke, **_: got.append(
+        (kb.tolist(), ke.tolist())))
+    q = torch.zeros((1, 1, 128), dtype=torch.bfloat16)
+    kv.ring_attention_fp8(q, None, None, None, None, None, kv_len, R, max_q_per_seq=1, single_launch=single_launch)
+    n = lens.tolist()
+    assert got == [([x * r // R for x in n], [x * (r + 1) // R for x in n]) for r in range(R)]

@@ -613,7 +613,8 @@ def ring_attention_fp8(q: torch.Tensor, cu_q: torch.Tensor, q_pos0: torch.Tensor
                                               N.stream_ptr(kv_len.device)), "ring_attention_fp8")
     else:
         steps = torch.arange(R + 1, dtype=torch.int64, device=kv_len.device)
-        bounds = kv_len.to(torch.int64)[None, :] * steps[:, None] // R
+        bounds = torch.empty((R + 1, B), dtype=torch.int32, device=kv_len.device)
+        bounds[:] = kv_len.to(torch.int64)[None, :] * steps[:, None] // R  # a [1, B] kv_len among others
         begin[:, :B], end[:, :B] = bounds[:-1], bounds[1:]
     if err is None:
         err = _err_word_if(check, q.device)
