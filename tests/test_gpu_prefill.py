@@ -66,6 +66,19 @@ def vmax_rows(pool, scales, bt, cu, kv_begin, kv_end, Hq):
     return out
 
 
+def kernels_of(fn):
+    """fn's result and the names of the kernels it launched, so that a test of one kernel
+    fails when the library's rule sends its call to another."""
+    for _ in range(3):  # (a first trace of a process may come back empty)
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            out = fn()
+            torch.cuda.synchronize()
+        names = " ".join(e.key for e in prof.key_averages())
+        if "kernel" in names:
+            break
+    return out, names
+
+
 P_BOUND = {"exact": (1, 2.0 ** -17), "f16": (2, 2.0 ** -10), "bf16": (2, 2.0 ** -7)}  # (ulps, bound on |V|)
 LSE_EXTRA = {"exact": 0.0, "f16": 2.0 ** -11 / np.log(2.0), "bf16": 2.0 ** -8 / np.log(2.0)}
 
@@ -534,15 +547,16 @@ def _f64_rows(q, pool, scales, bt, cu, qp, ranges, causal, sm):
     return out, vmax
 
 
-@pytest.mark.parametrize("case", ["causal", "full", "ring", "gaps", "large_scores", "bad_page"])
+@pytest.mark.parametrize("case", ["causal", "full", "ring", "gaps", "large_scores", "negative", "bad_page"])
 @pytest.mark.parametrize("precision", ["f16", "bf16"])
 def test_wide_prefill(case, precision):
     """The kernel with 64 rows per wave (four heads per KV head, at least a block per CU, room
     for 4,096 positions): ragged last tiles, steps cut by range ends, ranges that follow each
     other (walked as one) and ranges with gaps, running maxima that are outgrown again and
-    again, and a bad page.  Bound: this module's, against float64."""
+    again, negative scales of some heads' K and of others' V, and a bad page.  Bound: this
+    module's, against float64."""
     Hq, Hkv, P = 32, 8, 48 if case == "gaps" else 16
-    n_q, q_pos0, lens = [1030, 577, 1], [0, 700, 90], [1030, 1277, 91]
+    n_q, q_pos0, lens = [1030, 901, 1], [0, 700, 90], [1030, 1601, 91]
     print(f"wide prefill {case} {precision}", flush=True)
     q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, n_q, q_pos0, lens, seed=77)
     t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
@@ -551,6 +565,8 @@ def test_wide_prefill(case, precision):
     causal, sm = case != "full", float(np.float32(1.0 / np.sqrt(128)))
     if case == "large_scores":
         sm *= 12.0
+    if case == "negative":
+        scales *= np.array([[-1, 1, 1, -1, 1, 1, -1, 1], [1, -1, 1, -1, 1, 1, 1, -1]], np.float32)
     lens = np.asarray(lens)
     if case == "ring":
         ranges = [(lens * r // 5, lens * (r + 1) // 5) for r in range(5)]
@@ -566,14 +582,41 @@ def test_wide_prefill(case, precision):
                                     t(np.array([r[1] for r in ranges], np.int32)), check=True, precision=precision)
         ranges = [(np.array([0, 0, 0]), np.array([lens[0], 20 * P, lens[2]])),
                   (np.array([0, 21 * P, 0]), np.array([0, lens[1], 0]))]
-        got = kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, t(np.zeros((1, 3), np.int32)),
-                                      t(lens[None].astype(np.int32)), precision=precision)
+        kb, ke = t(np.zeros((1, 3), np.int32)), t(lens[None].astype(np.int32))
     else:
-        got = kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, t(np.array([r[0] for r in ranges], np.int32)),
-                                      t(np.array([r[1] for r in ranges], np.int32)), causal=causal, sm_scale=sm,
-                                      check=True, precision=precision)
+        kb, ke = (t(np.array([r[i] for r in ranges], np.int32)) for i in (0, 1))
+    got, names = kernels_of(lambda: kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, kb, ke, causal=causal,
+                                                            sm_scale=sm, check=case != "bad_page", precision=precision))
+    assert "paged_prefill_wide_kernel" in names
     want, vmax = _f64_rows(q, pool, scales, bt, cu, qp, ranges, causal, sm)
     assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy(), precision)
+
+
+@pytest.mark.parametrize("below", [6, 14, 20, 22, 24])
+def test_wide_prefill_weights_far_below_the_largest(below):
+    """One key whose score lies ``below`` log2 units above all 65,535 others: their weights,
+    subnormal in fp16 from 22 on (2^(7 - 22) < 2^-14), count in the row sums as they do in
+    P.V.  They are powers of two, so P is exact and the result is the exact value within an
+    ulp of bf16 (at 22 they are 1.6% of a row's sum, four ulps)."""
+    Hq, Hkv, P, n_keys, n_q = 32, 8, 16, 65536, 2112
+    g = torch.Generator(device=DEV).manual_seed(1)
+    pool = torch.zeros((n_keys // P, 2, Hkv, P, 128), dtype=torch.uint8, device=DEV)
+    pool[:, 1] = torch.where(torch.rand(pool[:, 1].shape, generator=g, device=DEV) < 0.5, 0x38, 0x30).to(torch.uint8)
+    pool[0, 0, :, 0, 0] = 0x38  # key 0: 1.0 in channel 0, as every query
+    q = torch.zeros((n_q, Hq, 128), dtype=torch.bfloat16, device=DEV)
+    q[..., 0] = 1.0
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    got, names = kernels_of(lambda: kv.ring_attention_fp8(
+        q, i32([0, n_q]), i32([n_keys - n_q]), pool, torch.ones((2, Hkv), device=DEV),
+        torch.arange(n_keys // P, dtype=torch.int32, device=DEV)[None], i32([n_keys]), 1, causal=False,
+        sm_scale=below * float(np.log(2.0)), max_q_per_seq=n_q))
+    assert "paged_prefill_wide_kernel" in names
+    v = pool[:, 1].view(torch.float8_e4m3fn).float().double().permute(1, 0, 2, 3).reshape(Hkv, n_keys, 128)
+    w = torch.full((n_keys,), 2.0 ** -below, dtype=torch.float64, device=DEV)
+    w[0] = 1.0
+    want = (w[None, :, None] * v).sum(1) / w.sum()  # between 0.5 and 1: an ulp is 2^-8
+    diff = (got.double() - want.repeat_interleave(Hq // Hkv, 0)[None]).abs().max().item()
+    assert diff <= 2.0 ** -8, diff
 
 
 @pytest.mark.parametrize("Hq,Hkv,P,n_q,q_pos0,causal,precision", [
