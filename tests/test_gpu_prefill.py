@@ -592,6 +592,28 @@ def test_wide_prefill(case, precision):
     assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy(), precision)
 
 
+def test_wide_prefill_flags_rows_beyond_max_q_per_seq():
+    """As test_prefill_flags_rows_beyond_max_q_per_seq, for the 64-row kernel, whose last tile
+    would hold 32 rows more: the rows up to a multiple of 32 are computed (as by the 32-row
+    kernel), the others are left unwritten, and flagged."""
+    Hq, Hkv, P, n = 32, 8, 16, 1088
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, [n, n], [0, 0], [n, n], seed=79)
+    wide_bt = np.zeros((2, 4096 // P), np.int32)
+    wide_bt[:, :bt.shape[1]] = bt
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    args = (q.to(DEV), t(cu), t(qp), t(pool), t(scales), t(wide_bt), t(np.zeros(2, np.int32)), t(np.full(2, n, np.int32)))
+    want = kv.paged_attention_prefill(*args, max_q_per_seq=n, check=True)
+    out = torch.full(q.shape, 7.0, dtype=torch.bfloat16, device=DEV)
+    _, names = kernels_of(lambda: kv.paged_attention_prefill(*args, out=out, max_q_per_seq=n - 32))
+    assert "paged_prefill_wide_kernel" in names
+    for rows in (slice(0, n), slice(n, 2 * n)):
+        assert torch.equal(out[rows][:n - 32], want[rows][:n - 32]) and (out[rows][n - 32:] == 7.0).all()
+    for most, flagged in ((n - 32, True), (n - 31, False)):
+        err = torch.zeros(1, dtype=torch.int32, device=DEV)
+        kv.paged_attention_prefill(*args, max_q_per_seq=most, err=err)
+        assert bool(err.item() & kv.N.ZX_KERR_POS_RANGE) == flagged
+
+
 @pytest.mark.parametrize("below", [6, 14, 20, 22, 24])
 def test_wide_prefill_weights_far_below_the_largest(below):
     """One key whose score lies ``below`` log2 units above all 65,535 others: their weights,

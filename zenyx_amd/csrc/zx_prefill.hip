@@ -53,6 +53,7 @@ struct PrefillArgs {
   int64_t n_pages;
   int32_t n_q_heads, n_kv_heads, page_size, max_blocks, mode, causal, n_ranges, n_seqs;
   int32_t n_qt;  // query tiles per sequence (the grid is n_qt x n_split x head groups x sequences)
+  int64_t max_rows;     // rows of a sequence that are computed: max_q_per_seq up to a multiple of 128 / G
   int32_t n_split;      // blocks that share a query tile's keys; each writes a part of its own:
   int64_t part_stride;  // rows (x heads) between the parts in o_acc / lse2
   uint32_t p_magic;
@@ -165,8 +166,8 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
   const int64_t v_off = (int64_t)a.n_kv_heads * a.page_size * D;
   const int32_t *bt = a.bt + (int64_t)b * a.max_blocks;
   int32_t e = 0;
-  // rows past n_qt * QT (max_q_per_seq too small) are not computed: flag it
-  if (qt_rev == 0 && (int64_t)a.n_qt * QT < n_qb) e |= ZX_KERR_POS_RANGE;
+  // rows past max_rows (n_qt tiles; max_q_per_seq too small) are not computed: flag it
+  if (qt_rev == 0 && a.max_rows < n_qb) e |= ZX_KERR_POS_RANGE;
   const int kmax = a.max_blocks * a.page_size;  // < 2^31 (checked by the host)
   // keys past the block's last query position never count when causal
   const int last_row = min(row0_blk + QT, n_qb) - 1;
@@ -748,7 +749,9 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
   asm volatile("" ::"s"(cq0), "s"(cq1), "s"(qp0_32), "s"(kb0), "s"(ke0), "s"(sk), "s"(sv));
   const int64_t qp0 = qp0_32;
   const int64_t q_lo = cq0;
-  const int n_qb = cq1 - cq0;
+  // rows past max_rows (max_q_per_seq too small) are not computed: flagged below
+  const bool rows_left_out = a.max_rows < cq1 - cq0;
+  const int n_qb = rows_left_out ? (int)a.max_rows : cq1 - cq0;
   const int64_t row0_64 = ((int64_t)a.n_qt - 1 - qt_rev) * QT;
   if (row0_64 >= n_qb) return;
   const int row0_blk = (int)row0_64;
@@ -758,7 +761,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
   const int64_t v_off = (int64_t)a.n_kv_heads * a.page_size * D;
   const int32_t *bt = a.bt + (int64_t)b * a.max_blocks;
   int32_t e = 0;
-  if (qt_rev == 0 && (int64_t)a.n_qt * QT < n_qb) e |= ZX_KERR_POS_RANGE;
+  if (qt_rev == 0 && rows_left_out) e |= ZX_KERR_POS_RANGE;
   const int kmax = a.max_blocks * a.page_size;
   const int last_row = min(row0_blk + QT, n_qb) - 1;
   // Range r of this sequence: keys [kb, ke) (ke clipped to the block table), walked in
@@ -1401,6 +1404,7 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
   }
   const int QT = p.wide ? PW_ROWS : 32 * 4 / G;
   a.n_qt = (int32_t)ceil_div(max_q_per_seq, QT);
+  a.max_rows = ceil_div(max_q_per_seq, 128 / G) * (128 / G);  // (a wide block's 64 rows may hold fewer)
   const int64_t n_blocks = (int64_t)a.n_qt * p.n_split * (n_q_heads / G) * n_seqs;
   ZX_REQUIRE(n_blocks < (1LL << 31), "paged_attention_prefill: too many query tiles or sequences");
   const dim3 grid((unsigned)n_blocks);
