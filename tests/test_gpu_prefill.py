@@ -614,6 +614,33 @@ def test_wide_prefill_flags_rows_beyond_max_q_per_seq():
         assert bool(err.item() & kv.N.ZX_KERR_POS_RANGE) == flagged
 
 
+def test_wide_prefill_nan_v_reaches_no_further_than_the_32_row_kernels():
+    """A NaN V code at key k makes its channel NaN in the rows from k on, and may do so in rows
+    before it whose 32-row tile reaches the 64-key step that holds k.  Query positions start
+    at 16, so that the first half of a 64-row tile ends before a step that its second half
+    reaches."""
+    Hq, Hkv, P, n, at = 32, 8, 16, 1088, 16
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, [n, n], [at, at], [at + n, at + n], seed=80)
+    planted = {3: 100, 5: 127, 7: 500, 9: 1023, 11: 64}  # channel -> key, of sequence 0's KV head 2
+    for ch, k in planted.items():
+        pool[bt[0, k // P], 1, 2, k % P, ch] = 0x7F
+    wide_bt = np.zeros((2, 4096 // P), np.int32)
+    wide_bt[:, :bt.shape[1]] = bt
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    got, names = kernels_of(lambda: kv.paged_attention_prefill(
+        q.to(DEV), t(cu), t(qp), t(pool), t(scales), t(wide_bt), t(np.zeros(2, np.int32)),
+        t(np.full(2, at + n, np.int32)), max_q_per_seq=n))
+    assert "paged_prefill_wide_kernel" in names
+    nan = torch.isnan(got.float()).cpu().numpy()
+    row = np.arange(n)
+    may = np.zeros_like(nan)
+    for ch, k in planted.items():
+        assert nan[:n][row + at >= k][:, 8:12, ch].all()
+        reaches = at + np.minimum(row // 32 * 32 + 31, n - 1) >= k // 64 * 64
+        may[:n, 8:12, ch] = reaches[:, None]
+    assert not (nan & ~may).any(), np.argwhere(nan & ~may)[:5]
+
+
 @pytest.mark.parametrize("below", [6, 14, 20, 22, 24])
 def test_wide_prefill_weights_far_below_the_largest(below):
     """One key whose score lies ``below`` log2 units above all 65,535 others: their weights,

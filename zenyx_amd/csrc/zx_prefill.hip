@@ -963,15 +963,31 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
   };
   const int lim[2] = {row_lim(wrow0 + n), row_lim(wrow0 + 32 + n)};
   const int s_full = all_ok && qs >= 0.0f ? row_lim(wrow0) - (PF_KEYS - 1) : -1;
+  // P.V of a step that starts past the last key of the first 32 rows leaves them out: their
+  // weights are 0, and a NaN V there would reach rows up to 126 positions before its key
+  // instead of 94 (the 32-row kernel does not walk such steps for these rows)
+  const int lim_first = row_lim(wrow0 + 31);
+  bool pv_both = true;  // the step whose P.V is next has keys for the first 32 rows
   att_u32x4 kf[FD + 1], vf[FD + 1];
-  auto pv_tile = [&](int t) {
+  auto pv_tile = [&](int t, int rg0 = 0) {
     const att_u32x4 av = vf[t % (FD + 1)];
     const int kc = t >> 2, ct = t & 3;
 #pragma unroll
-    for (int rg = 0; rg < 2; ++rg) {
+    for (int rg = rg0; rg < 2; ++rg) {
       if constexpr (F16) o[rg][ct] = pw_mfma_f16(av, ph[rg][kc], o[rg][ct]);
       else o[rg][ct] = pw_mfma_bf16(av, ph[rg][kc], o[rg][ct]);
     }
+  };
+  auto pv_rest = [&](int vrd) {  // tiles whose first FD operands are read
+    auto tiles = [&](int rg0) {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        if (t + FD < 16) vf[(t + FD) % (FD + 1)] = ld_v(vrd, t + FD);
+        pv_tile(t, rg0);
+      }
+    };
+    if (pv_both) tiles(0);
+    else tiles(1);
   };
   using Scores = att_f32x16[2][2];  // [rg][KT]
   // word w of the weights of key chunk kc as 16-bit pairs, and the chunk's sum
@@ -1041,6 +1057,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
     for (int rg = 0; rg < 2; ++rg)
 #pragma unroll
       for (int kc = 0; kc < 4; ++kc) ph[rg][kc] = att_u32x4{0u, 0u, 0u, 0u};
+    pv_both = true;
     __syncthreads();
     int kbuf = 0, vrd = 3 * PW_VBYTES, vnext = PW_VBYTES;
 #pragma unroll
@@ -1115,14 +1132,11 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
         for (int t = 0; t < FD; ++t) vf[t] = ld_v(vrd, t);
         __syncthreads();
         issue_step(j + 2, cb);
-#pragma unroll
-        for (int t = 0; t < 16; ++t) {
-          if (t + FD < 16) vf[(t + FD) % (FD + 1)] = ld_v(vrd, t + FD);
-          pv_tile(t);
-        }
+        pv_rest(vrd);
       }
       {
         const bool full = s0 >= g.kb && s0 <= s_hi;
+        pv_both = s0 <= lim_first;
         // the step with its running maxima looked at and the masks applied: the first step, the
         // steps that cross a boundary, and one whose weights outgrew the maxima (its S^T made
         // again; this step's K is still in LDS)
@@ -1193,11 +1207,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
     // P.V of the last step
 #pragma unroll
     for (int t = 0; t < FD; ++t) vf[t] = ld_v(vrd, t);
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      if (t + FD < 16) vf[(t + FD) % (FD + 1)] = ld_v(vrd, t + FD);
-      pv_tile(t);
-    }
+    pv_rest(vrd);
     rc = next_range(rc + 1, g);
     if (rc < n_ranges) {
       fill_table(0);
