@@ -602,12 +602,15 @@ def test_wide_prefill_flags_rows_beyond_max_q_per_seq():
     wide_bt[:, :bt.shape[1]] = bt
     t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
     args = (q.to(DEV), t(cu), t(qp), t(pool), t(scales), t(wide_bt), t(np.zeros(2, np.int32)), t(np.full(2, n, np.int32)))
-    want = kv.paged_attention_prefill(*args, max_q_per_seq=n, check=True)
+    want, vmax = _f64_rows(args[0], args[3], args[4], args[5], cu, qp, [([0, 0], [n, n])], True,
+                           float(np.float32(1.0 / np.sqrt(128))))
     out = torch.full(q.shape, 7.0, dtype=torch.bfloat16, device=DEV)
     _, names = kernels_of(lambda: kv.paged_attention_prefill(*args, out=out, max_q_per_seq=n - 32))
     assert "paged_prefill_wide_kernel" in names
-    for rows in (slice(0, n), slice(n, 2 * n)):
-        assert torch.equal(out[rows][:n - 32], want[rows][:n - 32]) and (out[rows][n - 32:] == 7.0).all()
+    for at in (0, n):
+        rows = slice(at, at + n - 32)
+        assert_precision(bits16(out[rows]), bits16(want[rows].to(torch.bfloat16)), vmax[rows].cpu().numpy())
+        assert (out[at + n - 32:at + n] == 7.0).all()
     for most, flagged in ((n - 32, True), (n - 31, False)):
         err = torch.zeros(1, dtype=torch.int32, device=DEV)
         kv.paged_attention_prefill(*args, max_q_per_seq=most, err=err)
@@ -639,6 +642,44 @@ def test_wide_prefill_nan_v_reaches_no_further_than_the_32_row_kernels():
         reaches = at + np.minimum(row // 32 * 32 + 31, n - 1) >= k // 64 * 64
         may[:n, 8:12, ch] = reaches[:, None]
     assert not (nan & ~may).any(), np.argwhere(nan & ~may)[:5]
+
+
+def test_wide_prefill_keys_above_the_first_ones():
+    """All keys but the first 64 score 6 log2 units above those: within the slack of a running
+    maximum, but the sums of their weights are not.  The maxima follow, so the call takes no
+    longer than with the keys 1 above (every step was made twice where they did not: 1.6
+    times), and the rows are the weighted means."""
+    Hq, Hkv, P, n = 32, 8, 16, 4096
+    g = torch.Generator(device=DEV).manual_seed(4)
+    pool = torch.zeros((2 * n // P, 2, Hkv, P, 128), dtype=torch.uint8, device=DEV)
+    pool[:, 1] = torch.where(torch.rand(pool[:, 1].shape, generator=g, device=DEV) < 0.5, 0x38, 0x30).to(torch.uint8)
+    pool[:, 0, :, :, 0] = 0x38
+    bt = torch.arange(2 * n // P, dtype=torch.int32, device=DEV).view(2, -1)
+    pool[bt[:, :4].flatten().long(), 0] = 0
+    q = torch.zeros((2 * n, Hq, 128), dtype=torch.bfloat16, device=DEV)
+    q[..., 0] = 1.0
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    args = (q, i32([0, n, 2 * n]), i32([0, 0]), pool, torch.ones((2, Hkv), device=DEV), bt, i32([[0, 0]]), i32([[n, n]]))
+    v = pool[bt.long(), 1].view(torch.float8_e4m3fn).float().double()  # [2, pages, Hkv, P, 128]
+    v = v.permute(0, 2, 1, 3, 4).reshape(2, Hkv, n, 128)
+    took = {}
+    for above in (1, 6, 1, 6):
+        call = lambda: kv.paged_attention_ring(*args, causal=False, sm_scale=above * float(np.log(2.0)), max_q_per_seq=n)  # noqa: E731,B023
+        got, names = kernels_of(call)
+        assert "paged_prefill_wide_kernel" in names
+        w = torch.ones(n, dtype=torch.float64, device=DEV)
+        w[:64] = 2.0 ** -above
+        want = ((w[None, None, :, None] * v).sum(2) / w.sum()).repeat_interleave(Hq // Hkv, 1)  # [2, Hq, 128]
+        assert (got.view(2, n, Hq, 128).double() - want[:, None]).abs().max() <= 2.0 ** -8
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            call()
+            b.record()
+            b.synchronize()
+            took[above] = min(took.get(above, 1e9), a.elapsed_time(b))
+    print(f"1 above: {took[1] * 1e3:.0f} us, 6 above: {took[6] * 1e3:.0f} us", flush=True)
+    assert took[6] <= 1.3 * took[1], took
 
 
 @pytest.mark.parametrize("below", [6, 14, 20, 22, 24])

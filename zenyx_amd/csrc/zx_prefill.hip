@@ -693,9 +693,12 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
 // work add up to what the vector unit can issue (a step of 64 keys: ~2,000 + ~2,000 cycles
 // measured for the two halves, 1,107 + 1,107 of them matrix time).
 // No running maximum is computed in these steps: the weights are taken under the maxima the
-// rows have, and only if a lane's sum shows that a score has outgrown them (2^PF_LAZY, as
-// above), or where masks apply or a row has no key yet, the step's S^T is made again and
-// the maxima are looked at (K has three buffers in LDS for that, V^T four: a wave may be one
+// rows have, and only if a lane's sum of 16 weights exceeds 2^PF_LAZY (a score has outgrown
+// its maximum by PF_LAZY, or many have by 4 and more), or where masks apply or a row has no
+// key yet, the step's S^T is made again and the maxima are looked at; a repeated step
+// raises every maximum that a score exceeds, after which no sum can trip the test until
+// scores grow again (4 x 8,192 causal, all keys but the first 64 at 6 above those: 3,430
+// us where only scores beyond PF_LAZY raised it, 2,081 so).  (K has three buffers in LDS for that, V^T four: a wave may be one
 // step ahead of another).  Looking at the maxima in every step cost 12% (2.17 against 2.10
 // ms); leaving its exponentials in one half of the step, with scalar page lookups between
 // the halves, 2.22 ms.
@@ -1174,7 +1177,9 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
           for (int i = 0; i < 32; i += 2) mx = fmaxf(fmaxf(mx, s[rg][i >> 4][i & 15]), s[rg][i >> 4][(i & 15) + 1]);
           xrow_pair32(mx * qe, x, y);
           const float w = fmaxf(x, y);
-          const bool grow = w > m[rg] + PF_LAZY;
+          // (after a repeat by as little as it takes: left where it is, a maximum 4 to 8 below
+          // the scores would have every further step repeated)
+          const bool grow = w > m[rg] + (grown ? 0.0f : PF_LAZY);
           const float mn = grow ? w : m[rg];
           const float ms = mn == -INFINITY ? 0.0f : mn;  // a row with no key yet keeps p = 0
           alpha[rg] = grow ? __builtin_amdgcn_exp2f(m[rg] - ms) : 1.0f;
