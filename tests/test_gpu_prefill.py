@@ -644,6 +644,39 @@ def test_wide_prefill_nan_v_reaches_no_further_than_the_32_row_kernels():
     assert not (nan & ~may).any(), np.argwhere(nan & ~may)[:5]
 
 
+def _least_us(call):
+    took = []
+    for _ in range(8):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        call()
+        b.record()
+        b.synchronize()
+        took.append(a.elapsed_time(b) * 1e3)
+    return min(took)
+
+
+@pytest.mark.parametrize("kind", ["negative_scale"])
+def test_wide_prefill_takes_the_overlapped_steps(kind):
+    """Calls that once sent every step through the kernel's masked path (1.9 times the time)
+    take no longer than the plain call."""
+    Hq, Hkv, P, n = 32, 8, 16, 4096
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, [n, n], [0, 0], [n, n], seed=81)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    args = [q.to(DEV), t(cu), t(qp), t(pool), t(scales), t(bt), t(np.zeros((1, 2), np.int32)),
+            t(np.full((1, 2), n, np.int32))]
+    sm = 1e-4  # scores of a few log2 units: no step is repeated
+
+    def call(sign=1.0):
+        return kv.paged_attention_ring(*args, causal=False, sm_scale=sign * sm, max_q_per_seq=n)
+
+    assert "paged_prefill_wide_kernel" in kernels_of(call)[1]
+    plain = min(_least_us(call), _least_us(call))
+    odd = min(_least_us(lambda: call(-1.0)), _least_us(lambda: call(-1.0)))
+    print(f"plain {plain:.0f} us, {kind} {odd:.0f} us", flush=True)
+    assert odd <= 1.3 * plain
+
+
 def test_wide_prefill_keys_above_the_first_ones():
     """All keys but the first 64 score 6 log2 units above those: within the slack of a running
     maximum, but the sums of their weights are not.  The maxima follow, so the call takes no
@@ -671,14 +704,8 @@ def test_wide_prefill_keys_above_the_first_ones():
         w[:64] = 2.0 ** -above
         want = ((w[None, None, :, None] * v).sum(2) / w.sum()).repeat_interleave(Hq // Hkv, 1)  # [2, Hq, 128]
         assert (got.view(2, n, Hq, 128).double() - want[:, None]).abs().max() <= 2.0 ** -8
-        for _ in range(8):
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record()
-            call()
-            b.record()
-            b.synchronize()
-            took[above] = min(took.get(above, 1e9), a.elapsed_time(b))
-    print(f"1 above: {took[1] * 1e3:.0f} us, 6 above: {took[6] * 1e3:.0f} us", flush=True)
+        took[above] = min(took.get(above, 1e9), _least_us(call))
+    print(f"1 above: {took[1]:.0f} us, 6 above: {took[6]:.0f} us", flush=True)
     assert took[6] <= 1.3 * took[1], took
 
 
