@@ -853,11 +853,11 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
   uint32_t tab_lo = 0, tab_hi = 0;
   int tab_n = 0;
   auto fill_table = [&](int base) {
-    const int64_t tp = (int64_t)g.s_first + (int64_t)(base + lane) * PF_KEYS + 16 * wave;
-    const int n_live = (int)max((int64_t)0, min((int64_t)16, g.ke - tp));
+    const int64_t at = (int64_t)g.s_first + (int64_t)(base + lane) * PF_KEYS, tp = at + 16 * wave;
+    const int n_live = at < g.ke_blk ? (int)max((int64_t)0, min((int64_t)16, g.ke - tp)) : 0;
     const uint32_t tc = n_live ? (uint32_t)tp : 0u;
     const uint32_t bi = pf_page_of(a, tc);
-    const int64_t page = n_live && g.s_first + (int64_t)(base + lane) * PF_KEYS < g.ke_blk ? bt[bi] : 0;
+    const int64_t page = n_live ? bt[bi] : 0;
     const bool ok = page >= 0 && page < a.n_pages;
     e |= ok ? 0 : ZX_KERR_PAGE_RANGE;
     const uint64_t off =
@@ -867,7 +867,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1) paged_prefill_wide_kernel(Prefi
     tab_n = ok ? n_live * D : 0;
   };
   const int ld_off = (kk0 & 15) * D + 16 * g8;
-  // K and V codes of step i of the range into registers (past its end: nothing is read)
+  // K and V codes of step i of the range into registers (past the block's last step: nothing
+  // is read)
   auto issue_step = [&](int i, Codes &c) {
     const uint64_t off = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)tab_lo, i & 63) |
                          (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)tab_hi, i & 63) << 32;
