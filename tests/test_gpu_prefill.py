@@ -767,6 +767,29 @@ def test_prefill_in_parts(Hq, Hkv, P, n_q, q_pos0, causal, precision):
         assert (out[int(cu[b]) + rows:int(cu[b]) + n] == 7.0).all()
 
 
+@pytest.mark.parametrize("ring", [8, 64])
+def test_parts_of_a_ring_are_equal(ring):
+    """The parts of a tile's keys are equal runs of all its steps, also where a ring's shards
+    have fewer steps than there are parts: such a ring takes about as long as one range (dealt
+    shard by shard, one part of a ring of 64 got every step: 3 times the time)."""
+    Hq, Hkv, P, n, old = 32, 8, 16, 64, 4032
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, [n], [old], [old + n], seed=82)
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    args = [q.to(DEV), t(cu), t(qp), t(pool), t(scales), t(bt)]
+    want, vmax = _f64_rows(args[0], args[3], args[4], args[5], cu, qp, [([0], [old + n])], True, 128 ** -0.5)
+    took = {}
+    for R in (1, ring, 1, ring):
+        kb, ke = (torch.arange(R, dtype=torch.int32, device=DEV)[:, None] + i for i in (0, 1))
+        kb, ke = kb * ((old + n) // R), ke * ((old + n) // R)
+        call = lambda: kv.paged_attention_ring(*args, kb, ke, max_q_per_seq=n)  # noqa: E731,B023
+        got, names = kernels_of(call)
+        assert "prefill_combine_kernel" in names
+        assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy())
+        took[R] = min(took.get(R, 1e9), _least_us(call))
+    print(f"one range {took[1]:.0f} us, ring of {ring} {took[ring]:.0f} us", flush=True)
+    assert took[ring] <= 1.6 * took[1]
+
+
 def test_ring_shard_bounds_match_torch():
     """The shard bounds' kernel against the integer expression, negative and large lengths
     among them; a kv_len of another dtype gives the same attention."""
