@@ -767,6 +767,45 @@ def test_prefill_in_parts(Hq, Hkv, P, n_q, q_pos0, causal, precision):
         assert (out[int(cu[b]) + rows:int(cu[b]) + n] == 7.0).all()
 
 
+@pytest.mark.parametrize("Hq,n_q,q_pos0,causal", [
+    (32, [64], [448], True),              # one part a tile: written by its own block
+    (32, [64, 64, 64, 64], [0] * 4, True),
+    (32, [70, 1, 33], [0, 3000, 900], True),  # one part, several, and in between
+    (16, [130, 40], [0, 2000], False),
+])
+def test_parts_follow_the_lengths(Hq, n_q, q_pos0, causal):
+    """A block table far wider than the sequences gives room for parts that the real lengths do
+    not need: the rows are right (in NaN-filled outputs), and the call takes about as long as
+    with the exact table (parts of the table's width: 5 times as long)."""
+    Hkv, P = 8, 16
+    lens = [p + n for p, n in zip(q_pos0, n_q)]
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, n_q, q_pos0, lens, seed=83)
+    wide_bt = np.full((len(lens), 32768 // P), -1, np.int32)
+    wide_bt[:, :bt.shape[1]] = bt
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    q, pool, scales = q.to(DEV), t(pool), t(scales)
+    zero, end = t(np.zeros(len(n_q), np.int32)), t(np.asarray(lens, np.int32))
+    want, vmax = _f64_rows(q, pool, scales, t(bt), cu, qp, [([0] * len(n_q), lens)], causal, 128 ** -0.5)
+    took = {}
+    for name, table in (("exact", t(bt)), ("wide", t(wide_bt))) * 2:
+        out = torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device=DEV)
+        call = lambda: kv.paged_attention_prefill(q, t(cu), t(qp), pool, scales, table, zero, end, causal=causal,  # noqa: E731,B023
+                                                  out=out, max_q_per_seq=max(n_q))  # noqa: B023
+        names = kernels_of(call)[1]
+        assert "prefill_combine_kernel" in names or name == "exact"
+        assert_precision(bits16(out), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy())
+        graph = torch.cuda.CUDAGraph()  # the launches without the host's part
+        args = (q, t(cu), t(qp), pool, scales, table, zero, end)
+        with torch.cuda.graph(graph):
+            for _ in range(10):
+                kv.paged_attention_prefill(*args, causal=causal, out=out, max_q_per_seq=max(n_q))
+        out.fill_(float("nan"))
+        took[name] = min(took.get(name, 1e9), _least_us(graph.replay) / 10)
+        assert_precision(bits16(out), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy())
+    print(f"exact table {took['exact']:.1f} us, 32k table {took['wide']:.1f} us", flush=True)
+    assert took["wide"] <= 1.4 * took["exact"] + 5
+
+
 @pytest.mark.parametrize("ring", [8, 64])
 def test_parts_of_a_ring_are_equal(ring):
     """The parts of a tile's keys are equal runs of all its steps, also where a ring's shards

@@ -56,6 +56,7 @@ struct PrefillArgs {
   int64_t max_rows;     // rows of a sequence that are computed: max_q_per_seq up to a multiple of 128 / G
   int32_t n_split;      // blocks that share a query tile's keys; each writes a part of its own:
   int64_t part_stride;  // rows (x heads) between the parts in o_acc / lse2
+  int32_t *parts;       // [n_qt x head groups x sequences] of them that a tile has
   uint32_t p_magic;
   int32_t p_shift;
   float sm_log2e;  // sm_scale * log2 e
@@ -112,6 +113,15 @@ __device__ __forceinline__ void decode16_f16(uint4 c, uint32_t (&b)[8]) {
   }
 }
 
+// Parts of a tile with `steps` steps: as many as the call has room for (the host knows the
+// width of the block table only), of at least 8 steps each.  Unused ones end at once, and a
+// tile of one part is written as if the call were not cut: 64 rows on 448 keys with a table
+// of 32,768 positions 127 -> 30 us (exact table 22), 4 x 64 rows of new sequences 54 -> 15
+// (exact table 11; the rest is the empty blocks and the second launch).
+__device__ __forceinline__ int pf_parts(int64_t steps, int n_split) {
+  return (int)max((int64_t)1, min((int64_t)n_split, steps / 8));
+}
+
 // PARTS: the blocks share each tile's keys (a.n_split > 1).  An instantiation of its own: the
 // extra live values cost the kernel without parts 3-7% (a ring of 8 launches over 4 x 8,192
 // rows 3,081 -> 3,297 us, exact weights 2,950 -> 3,054).
@@ -131,8 +141,6 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
   if constexpr (PARTS) {  // parts of one tile next to each other
     split = (int)(qt_rev % a.n_split);
     qt_rev /= a.n_split;
-    a.o_acc += split * a.part_stride * 128;
-    a.lse2 += split * a.part_stride;
   }
   const int hg = rem % n_hg, b = rem / n_hg;
   const int lane = threadIdx.x & 63;
@@ -237,8 +245,22 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
   if constexpr (PARTS) {
     int64_t total = 0;
     for (int r = 0; r < n_ranges; ++r) total += steps_of(range(r));
-    part_lo = total * split / a.n_split;
-    part_hi = total * (split + 1) / a.n_split;
+    const int parts = pf_parts(total, a.n_split);
+    if (split >= parts) {  // block-uniform exit
+      if (e && a.err && threadIdx.x == 0) atomicOr(a.err, e);
+      return;
+    }
+    if (split == 0 && threadIdx.x == 0) a.parts[qt_rev * per_rank + rem] = parts;
+    if (parts == 1) {  // the whole tile: its rows go to out, nothing is combined
+      a.mode = PF_WRITE_BF16;
+      part_hi = total;
+    } else {  // normalised rows and log2 sums of the part's own
+      a.mode = PF_MERGE | PF_INIT;
+      a.o_acc += split * a.part_stride * 128;
+      a.lse2 += split * a.part_stride;
+      part_lo = total * split / parts;
+      part_hi = total * (split + 1) / parts;
+    }
   }
   // range g, whose first step is step `before` of the tile, cut to this block's run
   auto cut = [&](Range &g, int64_t &before) {
@@ -1294,15 +1316,16 @@ constexpr int PC_MAX = 32;  // parts
 __global__ void __launch_bounds__(256) prefill_combine_kernel(PrefillArgs a, int32_t G, int32_t qt_rows) {
   const int n_hg = a.n_q_heads / G;
   const int64_t per_rank = (int64_t)n_hg * a.n_seqs;
-  const int64_t qt = (int64_t)blockIdx.x / per_rank;
-  const int rem = (int)((int64_t)blockIdx.x - qt * per_rank);
+  const int64_t qt_rev = (int64_t)blockIdx.x / per_rank;
+  const int rem = (int)((int64_t)blockIdx.x - qt_rev * per_rank);
   const int hg = rem % n_hg, b = rem / n_hg;
   const int32_t cq0 = a.cu_q[b], n_qb = a.cu_q[b + 1] - cq0;
-  const int64_t row0 = qt * qt_rows;
+  const int64_t row0 = ((int64_t)a.n_qt - 1 - qt_rev) * qt_rows;
   if (row0 >= n_qb) return;
   const int n_rows = (int)min((int64_t)qt_rows, n_qb - row0) * G;  // (row, head) pairs
   const int lane = threadIdx.x & 63, s_l = lane & 31;
-  const int S = a.n_split;
+  const int S = a.parts[blockIdx.x];
+  if (S == 1) return;  // its block has written the rows
   for (int i = threadIdx.x >> 5; i < n_rows; i += 8) {  // uniform in half a wave, where the shuffles stay
     const int64_t row = (cq0 + row0 + i / G) * a.n_q_heads + hg * G + i % G;
     const float ls = s_l < S ? a.lse2[s_l * a.part_stride + row] : -INFINITY;
@@ -1346,6 +1369,8 @@ namespace {
 struct PrefillPlan {
   int G, pm, n_split;
   bool wide;
+  int QT;           // rows per block
+  int64_t n_tiles;  // blocks that share no rows
 };
 PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int32_t page_size, int32_t max_blocks,
                          int32_t n_seqs, int32_t max_q_per_seq, int32_t causal, int32_t flags) {
@@ -1378,10 +1403,13 @@ PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int
     const int64_t parts = slots / nb >= 4 ? slots / nb : 2 * slots / nb;
     p.n_split = (int)std::max<int64_t>(1, std::min({parts, steps / 8, (int64_t)PC_MAX}));
   }
+  p.QT = p.wide ? PW_ROWS : 32 * 4 / p.G;
+  p.n_tiles = ceil_div(max_q_per_seq, p.QT) * (n_q_heads / p.G) * n_seqs;
   return p;
 }
 size_t prefill_part_bytes(const PrefillPlan &p, int64_t n_q, int32_t n_q_heads) {
-  return p.n_split > 1 ? (size_t)p.n_split * n_q * n_q_heads * (128 + 1) * sizeof(float) : 0;
+  return p.n_split > 1 ? (size_t)p.n_split * n_q * n_q_heads * (128 + 1) * sizeof(float) + p.n_tiles * sizeof(int32_t)
+                       : 0;
 }
 
 int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int32_t *q_pos0, int32_t n_q_heads,
@@ -1454,10 +1482,10 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
     a.p_shift = shift;
     a.p_magic = (uint32_t)(((1ULL << (31 + shift)) + page_size - 1) / page_size);
   }
-  const int QT = p.wide ? PW_ROWS : 32 * 4 / G;
+  const int QT = p.QT;
   a.n_qt = (int32_t)ceil_div(max_q_per_seq, QT);
   a.max_rows = ceil_div(max_q_per_seq, 128 / G) * (128 / G);  // (a wide block's 64 rows may hold fewer)
-  const int64_t n_blocks = (int64_t)a.n_qt * p.n_split * (n_q_heads / G) * n_seqs;
+  const int64_t n_blocks = p.n_tiles * p.n_split;
   ZX_REQUIRE(n_blocks < (1LL << 31), "paged_attention_prefill: too many query tiles or sequences");
   const dim3 grid((unsigned)n_blocks);
   hipStream_t st = as_stream(stream);
@@ -1468,10 +1496,10 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
   }
   a.n_split = p.n_split;
   a.part_stride = n_q * n_q_heads;
-  if (p.n_split > 1) {  // each part writes its own normalised rows and log2 sums
+  if (p.n_split > 1) {
     a.o_acc = static_cast<float *>(workspace);
     a.lse2 = a.o_acc + (int64_t)p.n_split * a.part_stride * 128;
-    a.mode = PF_MERGE | PF_INIT;
+    a.parts = reinterpret_cast<int32_t *>(a.lse2 + p.n_split * a.part_stride);
   }
   switch (G * 4 + pm) {
 #define ZX_PF_CASE(g, m)                                                                     \
@@ -1489,7 +1517,7 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
   }
   int rc = check_launch("paged_prefill_mfma");
   if (rc || p.n_split == 1) return rc;
-  prefill_combine_kernel<<<(unsigned)(n_blocks / p.n_split), 256, 0, st>>>(a, G, QT);
+  prefill_combine_kernel<<<(unsigned)p.n_tiles, 256, 0, st>>>(a, G, QT);
   return check_launch("prefill_combine");
 }
 }  // namespace
