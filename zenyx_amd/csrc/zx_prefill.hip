@@ -114,12 +114,13 @@ __device__ __forceinline__ void decode16_f16(uint4 c, uint32_t (&b)[8]) {
 }
 
 // Parts of a tile with `steps` steps: as many as the call has room for (the host knows the
-// width of the block table only), of at least 8 steps each.  Unused ones end at once, and a
-// tile of one part is written as if the call were not cut: 64 rows on 448 keys with a table
-// of 32,768 positions 127 -> 30 us (exact table 22), 4 x 64 rows of new sequences 54 -> 15
-// (exact table 11; the rest is the empty blocks and the second launch).
+// width of the block table only), of at least 2 steps each.  Unused ones end at once, and a
+// tile of one part is written as if the call were not cut.  With a table of 32,768 positions
+// (exact table in brackets): 64 rows on 448 keys 127 -> 20 us (22; 23 with parts of 4 steps,
+// 30 of 8), 16 x 4 rows on 500 19 (30), 4 x 64 rows of new sequences 54 -> 15 (11: the rest
+// is the empty blocks and the second launch).
 __device__ __forceinline__ int pf_parts(int64_t steps, int n_split) {
-  return (int)max((int64_t)1, min((int64_t)n_split, steps / 8));
+  return (int)max((int64_t)1, min((int64_t)n_split, steps / 2));
 }
 
 // PARTS: the blocks share each tile's keys (a.n_split > 1).  An instantiation of its own: the
@@ -1326,7 +1327,7 @@ __global__ void __launch_bounds__(256) prefill_combine_kernel(PrefillArgs a, int
   const int lane = threadIdx.x & 63, s_l = lane & 31;
   const int S = a.parts[blockIdx.x];
   if (S == 1) return;  // its block has written the rows
-  for (int i = threadIdx.x >> 5; i < n_rows; i += 8) {  // uniform in half a wave, where the shuffles stay
+  for (int i = 8 * blockIdx.y + (threadIdx.x >> 5); i < n_rows; i += 8 * gridDim.y) {  // uniform in half a wave, where the shuffles stay
     const int64_t row = (cq0 + row0 + i / G) * a.n_q_heads + hg * G + i % G;
     const float ls = s_l < S ? a.lse2[s_l * a.part_stride + row] : -INFINITY;
     float M = ls;
@@ -1517,7 +1518,10 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
   }
   int rc = check_launch("paged_prefill_mfma");
   if (rc || p.n_split == 1) return rc;
-  prefill_combine_kernel<<<(unsigned)p.n_tiles, 256, 0, st>>>(a, G, QT);
+  // a tile's 128 (row, head) pairs over up to 16 blocks (one block a tile: 64 rows on 8,128
+  // keys 81 us against 33, 2 x 300 on 4,000 113 against 90)
+  const unsigned gy = (unsigned)std::min<int64_t>(16, std::max<int64_t>(1, 8LL * num_cus() / p.n_tiles));
+  prefill_combine_kernel<<<dim3((unsigned)p.n_tiles, gy), 256, 0, st>>>(a, G, QT);
   return check_launch("prefill_combine");
 }
 }  // namespace
