@@ -234,3 +234,16 @@ def test_ring_shard_bounds_of_every_kv_len(monkeypatch, form, single_launch):
     kv.ring_attention_fp8(q, None, None, None, None, None, kv_len, R, max_q_per_seq=1, single_launch=single_launch)
     n = lens.tolist()
     assert got == [([x * r // R for x in n], [x * (r + 1) // R for x in n]) for r in range(R)]
+
+
+def test_prefill_plan_under_a_loose_bound():
+    """max_q_per_seq is a bound: one far above the call's rows gives the same plan (the same
+    workspace) as the number of its rows."""
+    from zenyx_amd import _native as N
+
+    size = N.load().zx_paged_attention_ring_workspace_bytes
+    for n_q, n_seqs, Hq, Hkv in ((64, 1, 32, 8), (256, 4, 32, 8), (33, 3, 8, 8), (700, 2, 16, 8)):
+        tight = size(n_q, Hq, Hkv, 16, 600, n_seqs, n_q, 1, N.ZX_PREFILL_BF16)
+        assert tight > 0
+        for most in (n_q + 1, 131072, 2**31 - 1):
+            assert size(n_q, Hq, Hkv, 16, 600, n_seqs, most, 1, N.ZX_PREFILL_BF16) == tight

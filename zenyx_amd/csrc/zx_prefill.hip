@@ -1371,11 +1371,16 @@ struct PrefillPlan {
   int G, pm, n_split;
   bool wide;
   int QT;           // rows per block
+  int32_t n_qt;     // tiles per sequence
+  int64_t max_rows; // rows per sequence that are computed (a wide block's 64 rows may hold fewer)
   int64_t n_tiles;  // blocks that share no rows
 };
 PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int32_t page_size, int32_t max_blocks,
                          int32_t n_seqs, int32_t max_q_per_seq, int32_t causal, int32_t flags) {
   PrefillPlan p;
+  // a loose bound (a model's longest context) launches no tiles that no sequence can have: 64
+  // rows on 8,128 keys under a bound of 131,072 390 us, 36 so
+  max_q_per_seq = (int32_t)std::min<int64_t>(max_q_per_seq, n_q);
   const int grp = n_q_heads / n_kv_heads;
   p.G = grp % 4 == 0 ? 4 : (grp % 2 == 0 ? 2 : 1);
   p.pm = (flags & ZX_PREFILL_EXACT_P) ? PF_P_EXACT : ((flags & ZX_PREFILL_FAST_P) ? PF_P_BF16 : PF_P_F16);
@@ -1405,7 +1410,9 @@ PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int
     p.n_split = (int)std::max<int64_t>(1, std::min({parts, steps / 8, (int64_t)PC_MAX}));
   }
   p.QT = p.wide ? PW_ROWS : 32 * 4 / p.G;
-  p.n_tiles = ceil_div(max_q_per_seq, p.QT) * (n_q_heads / p.G) * n_seqs;
+  p.n_qt = (int32_t)ceil_div(max_q_per_seq, p.QT);
+  p.max_rows = ceil_div(max_q_per_seq, 128 / p.G) * (128 / p.G);
+  p.n_tiles = (int64_t)p.n_qt * (n_q_heads / p.G) * n_seqs;
   return p;
 }
 size_t prefill_part_bytes(const PrefillPlan &p, int64_t n_q, int32_t n_q_heads) {
@@ -1483,9 +1490,8 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
     a.p_shift = shift;
     a.p_magic = (uint32_t)(((1ULL << (31 + shift)) + page_size - 1) / page_size);
   }
-  const int QT = p.QT;
-  a.n_qt = (int32_t)ceil_div(max_q_per_seq, QT);
-  a.max_rows = ceil_div(max_q_per_seq, 128 / G) * (128 / G);  // (a wide block's 64 rows may hold fewer)
+  a.n_qt = p.n_qt;
+  a.max_rows = p.max_rows;
   const int64_t n_blocks = p.n_tiles * p.n_split;
   ZX_REQUIRE(n_blocks < (1LL << 31), "paged_attention_prefill: too many query tiles or sequences");
   const dim3 grid((unsigned)n_blocks);
@@ -1521,7 +1527,7 @@ int prefill_impl(const uint16_t *q, int64_t n_q, const int32_t *cu_q, const int3
   // a tile's 128 (row, head) pairs over up to 16 blocks (one block a tile: 64 rows on 8,128
   // keys 81 us against 33, 2 x 300 on 4,000 113 against 90)
   const unsigned gy = (unsigned)std::min<int64_t>(16, std::max<int64_t>(1, 8LL * num_cus() / p.n_tiles));
-  prefill_combine_kernel<<<dim3((unsigned)p.n_tiles, gy), 256, 0, st>>>(a, G, QT);
+  prefill_combine_kernel<<<dim3((unsigned)p.n_tiles, gy), 256, 0, st>>>(a, G, p.QT);
   return check_launch("prefill_combine");
 }
 }  // namespace
