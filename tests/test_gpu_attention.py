@@ -166,3 +166,34 @@ def test_paged_attention_decode_runs_and_segments(dev, Hq, Hkv, D, P, lens):
                                     torch.from_numpy(bt).to(dev), torch.from_numpy(lens).to(dev), check=True)
     assert_within_one_ulp(bits16(got), want, v_colmax(pool, scales, bt, lens, Hq))
     assert not bits16(got)[lens == 0].any()
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(8, 8), (16, 8), (32, 8), (128, 8)])
+def test_decode_head_dim_64_weights_keep_32_bits(dev, Hq, Hkv):
+    """Pairs of keys whose weights differ by 2^-13 with values +448 and -448: the values cancel,
+    and what is left shows the error of the weights.  With 32-bit weights and products it
+    is at most that of exp2 (an ulp), of its argument (below 4, rounded to 2^-23) and of
+    the sums, 2^-20.5 max|V| together; weights in two bf16 terms give 2^-18.7."""
+    B, n, D, P = 64, 8, 64, 16
+    g = torch.Generator().manual_seed(Hq)
+    k = torch.zeros((B, Hkv, P, D))
+    k[..., 0] = torch.randint(-8, 9, (B, Hkv, P // 2), generator=g).repeat_interleave(2, 2) / 8.0  # e4m3 values
+    k[..., 1::2, 1] = 1.0
+    v = torch.randint(0, 2, (B, Hkv, P // 2, D), generator=g).repeat_interleave(2, 2) * 2.0 - 1.0
+    v[..., 1::2, :] *= -1.0
+    pool = torch.stack([k, 448.0 * v], 1).to(torch.float8_e4m3fn).view(torch.uint8)  # a page per sequence
+    q = torch.zeros((B, Hq, D))
+    q[..., 0] = torch.rand((B, Hq), generator=g) * 4.0 - 2.0
+    q[..., 1] = 2.0 ** -13
+    q = q.to(torch.bfloat16)
+    got = kv.paged_attention_decode(q.to(dev), pool.to(dev), torch.ones((2, Hkv), device=dev),
+                                    torch.arange(B, dtype=torch.int32, device=dev)[:, None].contiguous(),
+                                    torch.full((B,), n, dtype=torch.int32, device=dev), sm_scale=1.0)
+    rep = Hq // Hkv
+    kd, vd = (t[:, :, :n].double().repeat_interleave(rep, 1) for t in (k, 448.0 * v))
+    w = torch.softmax((q.double()[:, :, None] * kd).sum(-1), -1)
+    want = (w[..., None] * vd).sum(2)
+    off = (got.cpu().double() - want).abs() - want.abs() * 2.0 ** -8  # the rounding to bf16: half an ulp
+    worst = off.max().item() / 448.0
+    print(f"Hq {Hq}: 2^{np.log2(max(worst, 1e-12)):.1f} max|V|", flush=True)
+    assert worst <= 2.0 ** -20.5

@@ -464,8 +464,11 @@ paged_decode_partial_kernel(const uint16_t *__restrict__ q, AttnGeom g, const ui
 //     operand of P.V (8 consecutive tokens of one channel per lane) comes back through
 //     gfx950's transposing LDS read, ds_read_b64_tr_b16 (2% faster than storing V^T with
 //     64 two-byte stores per lane and step).
-// P goes through LDS as fp32 into the A-operand layout and is split into bf16 hi + lo
-// (two MFMAs), which keeps the products at ~2^-17 relative error.  Scores land in the C
+// P goes through LDS as fp32 into the A-operand layout and is split into bf16 terms: for
+// D = 128 hi + lo (two MFMAs), which keeps the products at ~2^-17 relative error; for D = 64
+// the rest as well (three MFMAs: all 24 bits of P, as in the fp32 products of the kernel
+// above: where values nearly cancel the error against 64 bits is 2^-24 max|V| as there, and
+// 2^-18.5 with two terms; 16 x 1k-8k, Hq 32 / Hkv 8: 24.2 us against 23.3).  Scores land in the C
 // layout: lane row kg (16 lanes) holds heads 4 kg ..+4 of token l % 16, so the softmax
 // bookkeeping is a 16-lane DPP reduction per head; the O accumulators (8 tiles of 16
 // channels) live in MFMA results, rows = heads.
@@ -494,6 +497,7 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
   constexpr int CPK = D / 4;     // channels per lane row kg of the q.K^T operands
   constexpr int NC = D / 32;     // q.K^T products per tile
   constexpr int NT = D / 16;     // 16-channel tiles of O
+  constexpr bool P3 = D == 64;   // P in three bf16 terms
   const int G = g.group;
   const int grp_blocks = g.n_q_heads / g.n_kv_heads / G;
   const int h = blockIdx.y / grp_blocks;
@@ -658,8 +662,8 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // A operand: P[head n][tokens 8 kg ..+8], split into bf16 hi + lo
-        att_bf16x8 ah, al;
+        // A operand: P[head n][tokens 8 kg ..+8], split into bf16 hi + lo (+ the rest)
+        att_bf16x8 ah, al, ar;
         {
           float pr[8];
           if (n < G) {
@@ -673,7 +677,9 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             ah[i] = (__bf16)pr[i];
-            al[i] = (__bf16)(pr[i] - (float)ah[i]);
+            const float rest = pr[i] - (float)ah[i];
+            al[i] = (__bf16)rest;
+            if constexpr (P3) ar[i] = (__bf16)(rest - (float)al[i]);
           }
         }
         // B operand per 16-channel tile: V^T[channel 16 jt + n][tokens 8 kg ..+8]
@@ -691,6 +697,7 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
                                     __builtin_bit_cast(uint2, w1).x, __builtin_bit_cast(uint2, w1).y});
           o[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bv, o[jt], 0, 0, 0);
           o[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bv, o[jt], 0, 0, 0);
+          if constexpr (P3) o[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ar, bv, o[jt], 0, 0, 0);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
