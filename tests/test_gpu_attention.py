@@ -28,6 +28,19 @@ def bf16_to_f32(b: np.ndarray) -> np.ndarray:
     return (b.astype(np.uint32) << 16).view(np.float32)
 
 
+def kernels_of(fn):
+    """fn's result and the names of the kernels it launched, so that a test of one kernel
+    fails when the library's rule sends its call to another."""
+    for _ in range(3):  # (a first trace of a process may come back empty)
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+            out = fn()
+            torch.cuda.synchronize()
+        names = " ".join(e.key for e in prof.key_averages())
+        if "kernel" in names:
+            break
+    return out, names
+
+
 def v_colmax(pool, scales, bt, lens, Hq):
     """max_t |V_t[d]| over each sequence's positions with a valid page: [B, Hq, D]."""
     n_pages, _, Hkv, P, D = pool.shape
@@ -197,3 +210,18 @@ def test_decode_head_dim_64_weights_keep_32_bits(dev, Hq, Hkv):
     worst = off.max().item() / 448.0
     print(f"Hq {Hq}: 2^{np.log2(max(worst, 1e-12)):.1f} max|V|", flush=True)
     assert worst <= 2.0 ** -20.5
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,kernel", [
+    (38, 2, 64, "partial"), (38, 2, 128, "partial"),  # 19 query heads per kv head: one per block
+    (8, 8, 64, "partial"), (36, 2, 64, "mfma"), (68, 2, 64, "mfma"), (26, 2, 128, "mfma"),  # 9, 2 and 13 per block
+])
+def test_decode_kernel_by_heads(dev, Hq, Hkv, D, kernel):
+    """The matrix-core kernel is for blocks of several query heads; one head per block goes to
+    the other.  Both against the oracle."""
+    q, pool, scales, bt, lens = make_case(Hq, Hkv, D, 16, [700, 17, 1], seed=Hq + D)
+    want, _ = O.paged_attention_decode(bits16(q), pool, scales, bt, lens, 1.0 / np.sqrt(D))
+    args = [t.to(dev) for t in (q, *map(torch.from_numpy, (pool, scales, bt, lens)))]
+    got, names = kernels_of(lambda: kv.paged_attention_decode(*args, check=True))
+    assert_within_one_ulp(bits16(got), want, v_colmax(pool, scales, bt, lens, Hq))
+    assert f"paged_decode_{kernel}_kernel" in names

@@ -23,7 +23,7 @@ import torch
 
 from oracle import oracle as O
 from zenyx_amd import kv
-from test_gpu_attention import assert_within_bound, bf16_to_f32
+from test_gpu_attention import assert_within_bound, bf16_to_f32, kernels_of
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
@@ -64,19 +64,6 @@ def vmax_rows(pool, scales, bt, cu, kv_begin, kv_end, Hq):
             h = hq // (Hq // Hkv)
             out[cu[b]:cu[b + 1], hq] = np.nanmax(dec[pool[pages, 1, h, t % P, :]], axis=0) * abs(float(scales[1, h]))
     return out
-
-
-def kernels_of(fn):
-    """fn's result and the names of the kernels it launched, so that a test of one kernel
-    fails when the library's rule sends its call to another."""
-    for _ in range(3):  # (a first trace of a process may come back empty)
-        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
-            out = fn()
-            torch.cuda.synchronize()
-        names = " ".join(e.key for e in prof.key_averages())
-        if "kernel" in names:
-            break
-    return out, names
 
 
 P_BOUND = {"exact": (1, 2.0 ** -17), "f16": (2, 2.0 ** -10), "bf16": (2, 2.0 ** -7)}  # (ulps, bound on |V|)

@@ -859,19 +859,21 @@ paged_decode_combine_kernel(const float *__restrict__ part, AttnGeom g, const fl
 
 using namespace zx;
 
-// The matrix-core variant (head_dim 64 and 128, pages of a multiple of 16) takes all query
-// heads of a kv head in one block, up to its 16 rows, so their pages are read once; with
-// one query head per kv head 15 of the 16 rows would be padding and the other variant is
-// faster (64 sequences of 2k-8k, 8 heads: D = 128 109 against 112 us, D = 64 59 against 69).
-// That one takes up to four heads per block.
-static bool att_mfma(int32_t grp, int32_t head_dim, int32_t page_size) {
-  return grp > 1 && head_dim <= 128 && page_size % 16 == 0;
-}
+// Query heads per block.  The matrix-core variant (head_dim 64 and 128, pages of a multiple of
+// 16) takes all query heads of a kv head in one block, up to its 16 rows, so their pages are
+// read once; with one head per block (one per kv head, or a prime number of more than 16) 15
+// of the 16 rows would be padding and the other variant is faster (64 sequences of 2k-8k, 8
+// heads: D = 128 109 against 112 us, D = 64 59 against 69; 16 x 1k-8k, 19 heads per kv head,
+// D = 64: 221 against 244, D = 128 371 against 384).  That one takes up to four heads per
+// block.
 static int32_t att_group(int32_t grp, bool mfma) {
   if (!mfma) return grp % 4 == 0 ? 4 : (grp % 2 == 0 ? 2 : 1);
   int g = grp < AM_ROWS ? grp : AM_ROWS;
   while (grp % g) --g;
   return g;
+}
+static bool att_mfma(int32_t grp, int32_t head_dim, int32_t page_size) {
+  return head_dim <= 128 && page_size % 16 == 0 && att_group(grp, true) > 1;
 }
 
 // The head_dims the kernels are built for; the plan below holds for these only.
