@@ -898,7 +898,19 @@ static AttnPlan att_plan(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads, 
   // resident blocks per group, one equal run each: two per CU (registers, and LDS at D = 128),
   // three where they fit (64 x 2k-8k, D = 64: 65 against 72 us).  More runs than resident
   // blocks leave a second, partly filled round: 16 x 1k-8k 37 against 31 us at three per CU.
-  const int64_t slots = std::max<int64_t>(1, (p.mfma && head_dim == 64 ? 3LL : 2LL) * num_cus() / groups);
+  // A number of groups that leaves a part of the CUs without a run takes up to four rounds of
+  // shorter ones where those fill the chip by 5% more (152 groups: 3 runs on 456 of 512, or 10
+  // in three rounds: 16 x 1k-8k, 19 heads per kv head, D = 128 371 -> 311 us, D = 64 221 -> 164).
+  const int64_t resident = (p.mfma && head_dim == 64 ? 3LL : 2LL) * num_cus();
+  int64_t slots = std::max<int64_t>(1, resident / groups);
+  double per_round = (double)slots;
+  for (int64_t rounds = 2; rounds <= 4; ++rounds) {
+    const int64_t n = rounds * resident / groups;
+    if ((double)n / rounds > 1.05 * per_round) {
+      slots = n;
+      per_round = (double)n / rounds;
+    }
+  }
   // one unit per sequence, or sequences of at most 512 positions that fill half the chip as
   // they are: whole sequences, no partials (32 x 100-500: 10.2 us, in runs 17)
   p.whole = seq_units == 1 || (seq_units * p.unit <= 512 && n_seqs >= slots / 2);
