@@ -23,7 +23,7 @@ import torch
 
 from oracle import oracle as O
 from zenyx_amd import kv
-from test_gpu_attention import assert_within_bound, bf16_to_f32, kernels_of
+from test_gpu_attention import assert_within_bound, bf16_to_f32, kernels_of, least_us
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda", 0)
@@ -631,18 +631,6 @@ def test_wide_prefill_nan_v_reaches_no_further_than_the_32_row_kernels():
     assert not (nan & ~may).any(), np.argwhere(nan & ~may)[:5]
 
 
-def _least_us(call):
-    took = []
-    for _ in range(8):
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        a.record()
-        call()
-        b.record()
-        b.synchronize()
-        took.append(a.elapsed_time(b) * 1e3)
-    return min(took)
-
-
 @pytest.mark.parametrize("kind", ["negative_scale"])
 def test_wide_prefill_takes_the_overlapped_steps(kind):
     """Calls that once sent every step through the kernel's masked path (1.9 times the time)
@@ -658,8 +646,8 @@ def test_wide_prefill_takes_the_overlapped_steps(kind):
         return kv.paged_attention_ring(*args, causal=False, sm_scale=sign * sm, max_q_per_seq=n)
 
     assert "paged_prefill_wide_kernel" in kernels_of(call)[1]
-    plain = min(_least_us(call), _least_us(call))
-    odd = min(_least_us(lambda: call(-1.0)), _least_us(lambda: call(-1.0)))
+    plain = min(least_us(call), least_us(call))
+    odd = min(least_us(lambda: call(-1.0)), least_us(lambda: call(-1.0)))
     print(f"plain {plain:.0f} us, {kind} {odd:.0f} us", flush=True)
     assert odd <= 1.3 * plain
 
@@ -691,7 +679,7 @@ def test_wide_prefill_keys_above_the_first_ones():
         w[:64] = 2.0 ** -above
         want = ((w[None, None, :, None] * v).sum(2) / w.sum()).repeat_interleave(Hq // Hkv, 1)  # [2, Hq, 128]
         assert (got.view(2, n, Hq, 128).double() - want[:, None]).abs().max() <= 2.0 ** -8
-        took[above] = min(took.get(above, 1e9), _least_us(call))
+        took[above] = min(took.get(above, 1e9), least_us(call))
     print(f"1 above: {took[1]:.0f} us, 6 above: {took[6]:.0f} us", flush=True)
     assert took[6] <= 1.3 * took[1], took
 
@@ -787,7 +775,7 @@ def test_parts_follow_the_lengths(Hq, n_q, q_pos0, causal):
             for _ in range(10):
                 kv.paged_attention_prefill(*args, causal=causal, out=out, max_q_per_seq=max(n_q))
         out.fill_(float("nan"))
-        took[name] = min(took.get(name, 1e9), _least_us(graph.replay) / 10)
+        took[name] = min(took.get(name, 1e9), least_us(graph.replay) / 10)
         assert_precision(bits16(out), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy())
     print(f"exact table {took['exact']:.1f} us, 32k table {took['wide']:.1f} us", flush=True)
     assert took["wide"] <= 1.1 * took["exact"] + 6
@@ -811,7 +799,7 @@ def test_parts_of_a_ring_are_equal(ring):
         got, names = kernels_of(call)
         assert "prefill_combine_kernel" in names
         assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy())
-        took[R] = min(took.get(R, 1e9), _least_us(call))
+        took[R] = min(took.get(R, 1e9), least_us(call))
     print(f"one range {took[1]:.0f} us, ring of {ring} {took[ring]:.0f} us", flush=True)
     assert took[ring] <= 1.6 * took[1]
 
