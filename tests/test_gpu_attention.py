@@ -259,3 +259,69 @@ def test_decode_four_heads_share_their_pages(dev, D, P):
         took[Hq] = least_us(lambda: kv.paged_attention_decode(*args))  # noqa: B023
     print(f"two heads {took[16]:.0f} us, four {took[32]:.0f} us", flush=True)
     assert took[32] <= 1.5 * took[16]
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,P", [(32, 8, 128, 16), (12, 12, 64, 16), (16, 4, 256, 8), (8, 2, 64, 24)])
+@pytest.mark.parametrize("lens", ["few_short", "few", "whole_64", "runs_64", "whole_65", "runs_65", "many_short",
+                                  "many", "one_long"])
+def test_decode_dealt_by_the_lengths(dev, Hq, Hkv, D, P, lens):
+    """The positions are dealt to the blocks in equal runs or as whole sequences, by the lengths
+    that the device reads (up to 64 sequences in every wave, more by a kernel of its own):
+    every way of it against the oracle, with empty sequences among them, and in a graph
+    that is replayed with other lengths."""
+    rng = np.random.default_rng(len(lens) + D)
+    n = {"few_short": rng.integers(0, 200, 5), "few": rng.integers(0, 3000, 9), "whole_64": rng.integers(0, 130, 64),
+         "runs_64": rng.integers(0, 700, 64), "whole_65": rng.integers(0, 130, 65), "runs_65": rng.integers(0, 700, 65),
+         "many_short": rng.integers(0, 40, 1500), "many": rng.integers(0, 300, 300),
+         "one_long": np.r_[rng.integers(0, 20, 40), 6000, rng.integers(0, 20, 90)]}[lens].astype(np.int32)
+    if lens.startswith("runs"):
+        n[7] = 5000  # the longest is far above an equal share
+    B, width = len(n), -(-6200 // P) if B_wide(lens) else -(-int(n.max() + 1) // P)
+    need = np.maximum(-(-n // P), 1)
+    pages = int(need.sum()) + 3
+    pool = rng.integers(0, 256, (pages, 2, Hkv, P, D), dtype=np.uint8)
+    pool[(pool & 0x7F) == 0x7F] = 0x3A
+    bt = np.full((B, width), -1, np.int32)
+    perm = rng.permutation(pages).astype(np.int32)
+    for b, first in enumerate(np.cumsum(need) - need):
+        bt[b, :need[b]] = perm[first:first + need[b]]
+    scales = rng.uniform(1e-3, 0.05, (2, Hkv)).astype(np.float32)
+    q = torch.from_numpy(rng.standard_normal((B, Hq, D)).astype(np.float32)).to(torch.bfloat16)
+    qd, pd, sd, bd, nd = (t.to(dev) for t in (q, *map(torch.from_numpy, (pool, scales, bt, n))))
+    other = np.minimum(n, rng.permutation(n)).astype(np.int32)  # within every sequence's pages
+    want = {}
+    for key, v in (("n", n), ("other", other)):
+        want[key], err = O.paged_attention_decode(bits16(q), pool, scales, bt, v, 1.0 / np.sqrt(D))
+        assert err == 0
+        got = kv.paged_attention_decode(qd, pd, sd, bd, torch.from_numpy(v).to(dev), check=True)
+        assert_within_one_ulp(bits16(got), want[key], v_colmax(pool, scales, bt, v, Hq))
+        assert not bits16(got)[v == 0].any()
+    out = torch.empty_like(qd)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kv.paged_attention_decode(qd, pd, sd, bd, nd, out=out)
+    for key, v in (("other", other), ("n", n), ("other", other)):
+        nd.copy_(torch.from_numpy(v))
+        out.fill_(float("nan"))
+        graph.replay()
+        assert_within_one_ulp(bits16(out), want[key], v_colmax(pool, scales, bt, v, Hq))
+
+
+def B_wide(lens):
+    """Lengths that the host, which knows the table's width only, cannot deal as whole sequences."""
+    return lens not in ("few", "many")
+
+
+def test_decode_work_grows_with_the_sequences(dev):
+    """4,096 sequences take about 16 times as long as 256 (57 times where every block went
+    over all lengths)."""
+    took = {}
+    for B in (256, 4096):
+        pages = B * 38
+        pool = torch.randint(0, 0x70, (pages, 2, 8, 16, 128), dtype=torch.uint8, device=dev)
+        args = [torch.randn((B, 32, 128), device=dev).to(torch.bfloat16), pool, torch.full((2, 8), 0.01, device=dev),
+                torch.arange(pages, dtype=torch.int32, device=dev).view(B, 38).repeat(1, 2),
+                torch.full((B,), 600, dtype=torch.int32, device=dev)]
+        took[B] = least_us(lambda: kv.paged_attention_decode(*args))  # noqa: B023
+    print(f"256: {took[256]:.0f} us, 4,096: {took[4096]:.0f} us", flush=True)
+    assert took[4096] <= 24 * took[256]

@@ -14,7 +14,11 @@
 // sequence and begin the next: each part of it that lies in one sequence is a segment, with
 // its own running softmax.  A segment that is a whole sequence is finished by its block;
 // others leave a partial (m, l, acc[D]) per query head in the workspace, and pass 2
-// (paged_decode_combine_kernel) merges a sequence's partials and writes bf16.
+// (paged_decode_combine_kernel) merges a sequence's partials and writes bf16.  Many short
+// sequences are dealt whole instead (att_take_whole).  Which it is, and where a run begins,
+// follows from the lengths on the device, not from the width of the block tables: up to 64
+// sequences every wave finds it in its lanes, for more paged_decode_plan_kernel writes it
+// into the workspace.
 //
 // paged_decode_partial_kernel (any head_dim and page size): lane l of a wave owns 16
 // channels (dc = l % LPT, LPT = D / 16 lanes per token) of token slot l / LPT, so K and V
@@ -26,11 +30,10 @@
 // matrix cores where its tiles fit.
 //
 // Bound by HBM reads of the codes (1 B per element) once contexts are long, by the chain of
-// a block's first loads before.  One layer, Hq 32 / Hkv 8, D = 128, pages of 16, whole
-// call, against fixed splits of at least 1,024 positions (most of them empty or alone in a
-// last round when lengths differ): 1 x 2,048 20.4 -> 9.5 us; 16 x 1k-8k 50 -> 30.7 us (3.9
-// TB/s); 64 x 512-4k 89 -> 59 us; 8 x 8k-32k 88 -> 55 us (5.0 TB/s); 64 x 32k 686 -> 682 us
-// (6.3 TB/s).
+// a block's first loads before.  One layer, Hq 32 / Hkv 8, D = 128, pages of 16, on the GPU,
+// against fixed splits of at least 1,024 positions (most of them empty or alone in a last
+// round when lengths differ): 1 x 2,048 20.8 -> 9.9 us; 16 x 1k-8k 50 -> 29 us (4.1 TB/s);
+// 64 x 512-4k 90 -> 59 us; 1,024 x 600 273 -> 225 us; 64 x 32k 673 -> 663 us (6.5 TB/s).
 #include <algorithm>
 
 #include "zx_attn_common.h"
@@ -44,10 +47,11 @@ constexpr int AM_ROWS = 16;  // query heads a block of the matrix-core variant c
 
 struct AttnGeom {
   int32_t n_q_heads, n_kv_heads, head_dim, page_size, max_blocks, n_seqs;
-  int32_t n_blk;        // blocks per head group
+  int32_t n_run;        // equal runs, one block per head group each
   uint32_t unit, cap;   // positions per unit (a power of two); positions a block table holds
-  int32_t whole;        // block x takes sequence x whole (n_blk == n_seqs) instead of an equal run
-  int32_t group;                // query heads per block
+  uint32_t tail;        // see att_take_whole
+  int32_t whole;        // every sequence is taken whole: known to the host
+  int32_t group, n_group;       // query heads per block; groups of them
   uint32_t p_magic;  // t / page_size = (t * p_magic) >> (31 + p_shift) for t < 2^31
   int32_t p_shift;
   int64_t n_pages;
@@ -66,14 +70,28 @@ __device__ __forceinline__ uint32_t att_units(const AttnGeom &g, int32_t len) {
   return (att_live_len(g, len) + (g.unit - 1)) / g.unit;  // unit: a power of two
 }
 
-// The U units of all sequences dealt to n_blk blocks: block x takes q = U / n_blk of them,
-// the first r = U % n_blk blocks one more.  T: 32 bits where U fits.
+// The U units of all sequences dealt to n_run runs: run x takes q = U / n_run of them, the
+// first r = U % n_run one more.  T: 32 bits where U fits.
 template <typename T> struct AttnDeal {
   T q, r;
-  __device__ AttnDeal(T U, T n_blk) : q(U / n_blk), r(U % n_blk) {}
+  __device__ AttnDeal(T q_, T r_) : q(q_), r(r_) {}
   __device__ T begin(T x) const { return x * q + min(x, r); }
-  __device__ T block_of(T u) const { return u < r * (q + 1) ? u / (q + 1) : r + (u - r * (q + 1)) / q; }
+  __device__ T run_of(T u) const { return u < r * (q + 1) ? u / (q + 1) : r + (u - r * (q + 1)) / q; }
 };
+
+// Whole sequences instead of equal runs?  A run starts anew in every sequence that it touches
+// (q, the first page ids, K and V one after the other: about as long as four units) and its
+// parts are merged; whole sequences leave blocks idle while the longest one ends.  With as many
+// sequences as runs or more, where most runs would start anew anyway: if the longest one has
+// at most ATT_TAIL_MANY positions and an eighth of an equal share.  Else if it exceeds a share
+// by at most ATT_TAIL_ONE units.  (g.tail: that slack in units; a call whose longest sequence
+// is within it needs no sums.)  In a graph, Hq 32 / Hkv 8, D = 128, tables of 32k positions:
+// 512 x 100-500 139 us in runs, 90 whole; 4 x 100-500 10.9 in runs, 16.3 whole; 64 x 512-4k
+// 59 in runs, 73 whole.
+constexpr uint32_t ATT_TAIL_ONE = 2, ATT_TAIL_MANY = 1024;
+__device__ __forceinline__ bool att_take_whole(const AttnGeom &g, uint64_t most, uint64_t share) {
+  return most <= g.tail + (g.n_seqs < g.n_run ? share : share / 8);
+}
 
 // Inclusive sum over the lanes below n (n <= 64, uniform).
 __device__ __forceinline__ uint32_t att_scan(uint32_t v, int n) {
@@ -85,84 +103,170 @@ __device__ __forceinline__ uint32_t att_scan(uint32_t v, int n) {
   return v;
 }
 
+// More than 64 sequences: what every block needs to know, computed once by att_plan_kernel.
+struct AttnTable {
+  uint64_t *head;   // [4]: whole sequences?, q, r
+  uint64_t *first;  // [n_seqs] a sequence's first unit
+  int32_t *x0, *n_live;  // [n_seqs] the first run that holds a part of it, and how many do
+  int32_t *run_b;        // [n_run] the sequence in which a run begins
+  __host__ __device__ AttnTable(void *at, int64_t n_seqs) {
+    head = static_cast<uint64_t *>(at);
+    first = head + 4;
+    x0 = reinterpret_cast<int32_t *>(first + n_seqs);
+    n_live = x0 + n_seqs;
+    run_b = n_live + n_seqs;
+  }
+  static size_t bytes(int64_t n_seqs, int64_t n_run) {
+    return 4 * sizeof(uint64_t) + (size_t)n_seqs * (sizeof(uint64_t) + 2 * sizeof(int32_t)) +
+           (size_t)n_run * sizeof(int32_t);
+  }
+};
+
 // The run of block x: units [u, u_end), unit u in sequence b, whose first unit is b_first.
 // All block-uniform; an empty run has u == u_end.  Up to 64 sequences every lane keeps one
 // sequence's length, so that stepping to the next sequence reads no memory.
 struct AttnRun {
   uint64_t u, u_end, b_first;
   int32_t b, lane_len;
+  int32_t x, y;  // the run (or sequence) and the group of query heads
 };
 __device__ __forceinline__ int32_t att_len(const AttnGeom &g, const int32_t *seq_lens, const AttnRun &r) {
   return g.n_seqs <= 64 ? __builtin_amdgcn_readlane(r.lane_len, r.b) : seq_lens[r.b];
 }
-__device__ __forceinline__ AttnRun att_locate(const AttnGeom &g, const int32_t *seq_lens, int x) {
+// Lane b's units, and how up to 64 sequences are dealt: whole, or units [begin(x), begin(x +
+// 1)) to run x, where incl is the inclusive sum over the sequences.
+struct AttnLanes {
+  uint32_t n, incl = 0;
+  bool whole;
+  AttnDeal<uint32_t> deal;
+  __device__ AttnLanes(const AttnGeom &g, int32_t lane_len) : n(att_units(g, lane_len)), deal(0, 0) {
+    whole = __ballot(n > g.tail) == 0;
+    if (whole) return;
+    incl = att_scan(n, g.n_seqs);
+    const uint32_t all = __builtin_amdgcn_readlane(incl, g.n_seqs - 1);
+    deal = AttnDeal<uint32_t>(all / (uint32_t)g.n_run, all % (uint32_t)g.n_run);
+    whole = __ballot(!att_take_whole(g, n, deal.q)) == 0;
+  }
+};
+// Block `at` of a one-dimensional grid: the groups of a run (or sequence) are neighbours, so
+// that blocks that read the same pages run together, and the blocks without one come last
+// (between the others they left three quarters of the CUs idle).
+__device__ __forceinline__ AttnRun att_locate(const AttnGeom &g, const int32_t *seq_lens, const AttnTable &t,
+                                              uint32_t at) {
   AttnRun r;
   const int lane = threadIdx.x & 63;
   r.lane_len = lane < g.n_seqs ? seq_lens[lane] : 0;
-  if (g.whole) {
-    r.b = x;
-    r.u = r.b_first = 0;
-    r.u_end = __builtin_amdgcn_readfirstlane(att_units(g, att_len(g, seq_lens, r)));
-    return r;
+  r.x = (int)(at / (uint32_t)g.n_group);
+  r.y = (int)(at - (uint32_t)r.x * (uint32_t)g.n_group);
+  const int x = r.x;
+  r.b = x;
+  r.u = r.u_end = r.b_first = 0;
+  bool whole = g.whole;
+  uint64_t q = 0, rem = 0;
+  if (!whole && g.n_seqs <= 64) {  // every wave by itself
+    const AttnLanes l(g, r.lane_len);
+    whole = l.whole;
+    if (!whole && x < g.n_run) {
+      const uint32_t u = l.deal.begin((uint32_t)x), u_end = l.deal.begin((uint32_t)x + 1);
+      r.u = u;
+      r.u_end = u_end;
+      const uint64_t after = __ballot(l.incl > u);  // sequences that end after u; the first holds it
+      r.b = after ? __ffsll((long long)after) - 1 : 0;
+      r.b_first = __builtin_amdgcn_readlane(l.incl - l.n, r.b);
+    }
+  } else if (!whole) {
+    whole = t.head[0] != 0;
+    q = t.head[1];
+    rem = t.head[2];
+    if (!whole && x < g.n_run) {
+      const AttnDeal<uint64_t> deal(q, rem);
+      r.u = deal.begin((uint64_t)x);
+      r.u_end = deal.begin((uint64_t)x + 1);
+      if (r.u < r.u_end) {
+        r.b = t.run_b[x];
+        r.b_first = t.first[r.b];
+      }
+    }
   }
-  if (g.n_seqs <= 64) {  // every wave by itself
-    const uint32_t n = att_units(g, r.lane_len);
-    const uint32_t incl = att_scan(n, g.n_seqs);
-    const AttnDeal<uint32_t> deal(__builtin_amdgcn_readlane(incl, g.n_seqs - 1), (uint32_t)g.n_blk);
-    const uint32_t u = deal.begin((uint32_t)x), u_end = deal.begin((uint32_t)x + 1);
-    r.u = u;
-    r.u_end = u_end;
-    const uint64_t after = __ballot(incl > u);  // sequences that end after u; the first holds it
-    r.b = after ? __ffsll((long long)after) - 1 : 0;
-    r.b_first = __builtin_amdgcn_readlane(incl - n, r.b);
-    return r;
-  }
-  // thread t sums sequences [t c, t c + c), a scan over the block gives each its first unit
-  __shared__ uint64_t wsum[ATT_WAVES], found_first;
-  __shared__ int32_t found_b;
-  const int wave = threadIdx.x >> 6;
-  const int c = (g.n_seqs + ATT_THREADS - 1) / ATT_THREADS;
-  const int b0 = min((int)threadIdx.x * c, g.n_seqs), b1 = min(b0 + c, g.n_seqs);
+  if (whole && x < g.n_seqs) r.u_end = __builtin_amdgcn_readfirstlane(att_units(g, att_len(g, seq_lens, r)));
+  return r;
+}
+
+// One block: the table of a call of more than 64 sequences.  (Each block of the two passes
+// scanned all lengths for itself before, work that grows with the square of the sequences:
+// 4,096 x 600 positions 4,580 us, 876 so.)
+constexpr int AP_THREADS = 1024;
+__global__ void __launch_bounds__(AP_THREADS)
+paged_decode_plan_kernel(AttnGeom g, const int32_t *__restrict__ seq_lens, void *table) {
+  const AttnTable t(table, g.n_seqs);
+  constexpr int WAVES = AP_THREADS / 64;
+  __shared__ uint64_t wsum[WAVES];
+  __shared__ uint32_t wmax[WAVES];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint64_t sum = 0;
-  for (int b = b0; b < b1; ++b) sum += att_units(g, seq_lens[b]);
-  uint64_t incl = sum;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint64_t y = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += y;
+  uint32_t most = 0;
+  for (int b = threadIdx.x; b < g.n_seqs; b += AP_THREADS) {
+    const uint32_t n = att_units(g, seq_lens[b]);
+    sum += n;
+    most = max(most, n);
   }
-  if (lane == 63) wsum[wave] = incl;
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    sum += __shfl_xor(sum, off, 64);
+    most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
+  }
+  if (lane == 0) wsum[wave] = sum, wmax[wave] = most;
   __syncthreads();
   uint64_t U = 0;
 #pragma unroll
-  for (int w = 0; w < ATT_WAVES; ++w) {
-    if (w < wave) incl += wsum[w];
+  for (int w = 0; w < WAVES; ++w) {
     U += wsum[w];
+    most = max(most, wmax[w]);
   }
-  const AttnDeal<uint64_t> deal(U, (uint64_t)g.n_blk);
-  r.u = deal.begin((uint64_t)x);
-  r.u_end = deal.begin((uint64_t)x + 1);
-  uint64_t first = incl - sum;
-  if (r.u < r.u_end && first <= r.u && r.u < incl) {  // one thread
-    int b = b0;
-    for (uint64_t n = att_units(g, seq_lens[b]); r.u >= first + n; n = att_units(g, seq_lens[b])) {
-      first += n;
-      ++b;
+  const AttnDeal<uint64_t> deal(U / (uint64_t)g.n_run, U % (uint64_t)g.n_run);
+  const bool whole = att_take_whole(g, most, deal.q);
+  if (threadIdx.x == 0) {
+    t.head[0] = whole;
+    t.head[1] = deal.q;
+    t.head[2] = deal.r;
+  }
+  uint64_t carry = 0;
+  for (int b0 = 0; b0 < g.n_seqs; b0 += AP_THREADS) {  // block-uniform
+    const int b = b0 + threadIdx.x;
+    const uint64_t n = b < g.n_seqs ? att_units(g, seq_lens[b]) : 0;
+    uint64_t incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint64_t y = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += y;
     }
-    found_b = b;
-    found_first = first;
+    __syncthreads();  // the sums of the round before have been read
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    uint64_t before = carry;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      if (w < wave) before += wsum[w];
+      carry += wsum[w];
+    }
+    if (b >= g.n_seqs) continue;
+    const uint64_t first = before + incl - n;
+    t.first[b] = first;
+    if (whole || n == 0) {
+      t.x0[b] = 0;
+      t.n_live[b] = n != 0;
+      continue;
+    }
+    const uint64_t xa = deal.run_of(first), xz = deal.run_of(first + n - 1);
+    t.x0[b] = (int32_t)xa;
+    t.n_live[b] = (int32_t)(xz - xa + 1);
+    for (uint64_t x = deal.begin(xa) < first ? xa + 1 : xa; x <= xz; ++x) t.run_b[x] = b;
   }
-  __syncthreads();
-  if (r.u < r.u_end) {
-    r.b = __builtin_amdgcn_readfirstlane(found_b);
-    r.b_first = found_first;
-  }
-  return r;
 }
 
 // Merges the block's four waves' (m, l, acc[G][D]) (in LDS, after a barrier) and stores the
 // segment's rows: bf16 rows when the segment is its whole sequence (zeros when no position
-// had a page), else partial x + b of the row's n_blk + n_seqs (moving along the runs, x or
+// had a page), else partial x + b of the row's n_run + n_seqs (moving along the runs, x or
 // b or both grow from one segment to the next, so x + b names a segment).
 template <int D, int ROWS>
 __device__ __forceinline__ void att_store(const AttnGeom &g, const float (&sm_m)[ATT_WAVES][ROWS],
@@ -185,7 +289,7 @@ __device__ __forceinline__ void att_store(const AttnGeom &g, const float (&sm_m)
       const float o = ll == 0.0f ? 0.0f : a / ll * sv;
       out[((int64_t)b * g.n_q_heads + hq0 + j) * D + d] = (uint16_t)(pack_bf16(o, 0.0f) & 0xFFFFu);
     } else {
-      float *pp = part + ((int64_t)(hq0 + j) * ((int64_t)g.n_blk + g.n_seqs) + x + b) * (2 + D);
+      float *pp = part + ((int64_t)(hq0 + j) * ((int64_t)g.n_run + g.n_seqs) + x + b) * (2 + D);
       pp[2 + d] = a;
       if (d == 0) {
         pp[0] = M;
@@ -233,20 +337,21 @@ template <int LPT> __device__ __forceinline__ float slots_sum(float v) {
   return rows_sum(v);
 }
 
-// Partial layout in the workspace: [Hq][n_blk + B][2 + D] fp32 = (m, l, acc[D]) with m in
+// Partial layout in the workspace: [Hq][n_run + B][2 + D] fp32 = (m, l, acc[D]) with m in
 // the exp2 domain; a segment without valid positions writes m = -inf, l = 0, acc = 0.
 template <int G, int D, bool FAST>
 __global__ void __launch_bounds__(ATT_THREADS)
 paged_decode_partial_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8_t *__restrict__ pool,
                             const float *__restrict__ scales, const int32_t *__restrict__ block_tables,
                             const int32_t *__restrict__ seq_lens, float *__restrict__ part,
-                            uint16_t *__restrict__ out, int32_t *err) {
+                            uint16_t *__restrict__ out, int32_t *err, void *table) {
   constexpr int LPT = D / 16;   // lanes per token
   constexpr int TPW = 64 / LPT;  // token slots per wave pass
   constexpr int STEP = ATT_U * TPW;
+  AttnRun run = att_locate(g, seq_lens, AttnTable(table, g.n_seqs), blockIdx.x);
   const int grp_blocks = g.n_q_heads / g.n_kv_heads / G;  // query-head groups per kv head
-  const int h = blockIdx.y / grp_blocks;
-  const int hq0 = h * (g.n_q_heads / g.n_kv_heads) + (blockIdx.y % grp_blocks) * G;
+  const int h = run.y / grp_blocks;
+  const int hq0 = h * (g.n_q_heads / g.n_kv_heads) + (run.y % grp_blocks) * G;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar addressing
   const int ts = lane / LPT, dc = lane % LPT;
@@ -257,7 +362,6 @@ paged_decode_partial_kernel(const uint16_t *__restrict__ q, AttnGeom g, const ui
   __shared__ float sm_m[ATT_WAVES][G], sm_l[ATT_WAVES][G];
   __shared__ float sm_acc[ATT_WAVES][G][D];
   int32_t e = 0;
-  AttnRun run = att_locate(g, seq_lens, blockIdx.x);
   if (g.whole && run.u == run.u_end) att_zero_rows(g, out, G, hq0, run.b, D);
   while (run.u < run.u_end) {
     const int b = run.b;
@@ -441,7 +545,7 @@ paged_decode_partial_kernel(const uint16_t *__restrict__ q, AttnGeom g, const ui
     __syncthreads();
     const float *const accs[ATT_WAVES] = {&sm_acc[0][0][0], &sm_acc[1][0][0], &sm_acc[2][0][0], &sm_acc[3][0][0]};
     if (t_begin < t_end)
-      att_store<D, G>(g, sm_m, sm_l, accs, part, out, G, hq0, b, blockIdx.x, whole_seq, scales[g.n_kv_heads + h]);
+      att_store<D, G>(g, sm_m, sm_l, accs, part, out, G, hq0, b, run.x, whole_seq, scales[g.n_kv_heads + h]);
     run.u = run.b_first + seg_end;
     run.b_first += b_units;
     ++run.b;
@@ -491,7 +595,7 @@ __global__ void __launch_bounds__(ATT_THREADS, 2)
 paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8_t *__restrict__ pool,
                          const float *__restrict__ scales, const int32_t *__restrict__ block_tables,
                          const int32_t *__restrict__ seq_lens, float *__restrict__ part,
-                         uint16_t *__restrict__ out, int32_t *err) {
+                         uint16_t *__restrict__ out, int32_t *err, void *table) {
   using Lds = AmLds<D>;
   constexpr int LPT = D / 16;   // lanes per token of a 16-byte load
   constexpr int TPL = 64 / LPT;  // tokens per load
@@ -501,9 +605,10 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
   constexpr int NT = D / 16;     // 16-channel tiles of O
   constexpr bool P3 = D == 64;   // P in three bf16 terms
   const int G = g.group;
+  AttnRun run = att_locate(g, seq_lens, AttnTable(table, g.n_seqs), blockIdx.x);
   const int grp_blocks = g.n_q_heads / g.n_kv_heads / G;
-  const int h = blockIdx.y / grp_blocks;
-  const int hq0 = h * (g.n_q_heads / g.n_kv_heads) + (blockIdx.y % grp_blocks) * G;
+  const int h = run.y / grp_blocks;
+  const int hq0 = h * (g.n_q_heads / g.n_kv_heads) + (run.y % grp_blocks) * G;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, kg = lane >> 4;  // MFMA column / k-group
@@ -517,7 +622,6 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
   float *pl = reinterpret_cast<float *>(lds[wave] + Lds::VBYTES);
   uint8_t *ks = lds[wave] + Lds::VBYTES + AM_PBYTES;
   int32_t e = 0;
-  AttnRun run = att_locate(g, seq_lens, blockIdx.x);
   if (g.whole && run.u == run.u_end) att_zero_rows(g, out, G, hq0, run.b, D);
   while (run.u < run.u_end) {
     const int b = run.b;
@@ -762,7 +866,7 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
     const float *const accs[ATT_WAVES] = {reinterpret_cast<const float *>(lds[0]), reinterpret_cast<const float *>(lds[1]),
                                           reinterpret_cast<const float *>(lds[2]), reinterpret_cast<const float *>(lds[3])};
     if (t_begin < t_end)
-      att_store<D, AM_ROWS>(g, sm_m, sm_l, accs, part, out, G, hq0, b, blockIdx.x, whole_seq, scales[g.n_kv_heads + h]);
+      att_store<D, AM_ROWS>(g, sm_m, sm_l, accs, part, out, G, hq0, b, run.x, whole_seq, scales[g.n_kv_heads + h]);
     run.u = run.b_first + seg_end;
     run.b_first += b_units;
     ++run.b;
@@ -780,49 +884,34 @@ paged_decode_mfma_kernel(const uint16_t *__restrict__ q, AttnGeom g, const uint8
 constexpr int CB_U = 8;  // segments whose values are loaded together
 __global__ void __launch_bounds__(256)
 paged_decode_combine_kernel(const float *__restrict__ part, AttnGeom g, const float *__restrict__ scales,
-                            const int32_t *__restrict__ seq_lens, uint16_t *__restrict__ out) {
+                            const int32_t *__restrict__ seq_lens, uint16_t *__restrict__ out, void *table) {
   const int D = g.head_dim;
   const int lane = threadIdx.x & 63;
   const int64_t row = blockIdx.x;  // b * Hq + hq
   const int d = threadIdx.x;
   const int b = (int)(row / g.n_q_heads);
   const int h = (int)(row % g.n_q_heads) / (g.n_q_heads / g.n_kv_heads);
-  // the sequence's first block, and how many hold a part of it
-  int64_t x0 = 0;
-  int n_live = 0;
+  // the sequence's first run, and how many hold a part of it
+  int32_t x0 = 0, n_live = 0;
   if (g.n_seqs <= 64) {
-    const uint32_t n = att_units(g, lane < g.n_seqs ? seq_lens[lane] : 0);
-    const uint32_t incl = att_scan(n, g.n_seqs);
-    const AttnDeal<uint32_t> deal(__builtin_amdgcn_readlane(incl, g.n_seqs - 1), (uint32_t)g.n_blk);
-    const uint32_t nb = __builtin_amdgcn_readlane(n, b), last = __builtin_amdgcn_readlane(incl, b) - 1;
-    if (nb) {
-      x0 = deal.block_of(last + 1 - nb);
-      n_live = (int)(deal.block_of(last) - x0 + 1);
+    const AttnLanes l(g, lane < g.n_seqs ? seq_lens[lane] : 0);
+    const uint32_t nb = __builtin_amdgcn_readlane(l.n, b);
+    if (l.whole) {
+      n_live = nb != 0;
+    } else if (nb) {
+      const uint32_t last = __builtin_amdgcn_readlane(l.incl, b) - 1;
+      x0 = (int32_t)l.deal.run_of(last + 1 - nb);
+      n_live = (int32_t)l.deal.run_of(last) - x0 + 1;
     }
   } else {
-    uint64_t first = 0, U = 0;
-    for (int b0 = 0; b0 < g.n_seqs; b0 += 64) {
-      const uint64_t n = b0 + lane < g.n_seqs ? att_units(g, seq_lens[b0 + lane]) : 0;
-      uint64_t a = n, c = b0 + lane < b ? n : 0;
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) {
-        a += __shfl_xor(a, off, 64);
-        c += __shfl_xor(c, off, 64);
-      }
-      U += a;
-      first += c;
-    }
-    const AttnDeal<uint64_t> deal(U, (uint64_t)g.n_blk);
-    const uint32_t nb = att_units(g, seq_lens[b]);
-    if (nb) {
-      x0 = (int64_t)deal.block_of(first);
-      n_live = (int)((int64_t)deal.block_of(first + nb - 1) - x0 + 1);
-    }
+    const AttnTable t(table, g.n_seqs);
+    x0 = t.x0[b];
+    n_live = t.n_live[b];
   }
   if (n_live == 1) return;  // the sequence was one segment: its block has written the row
   const float sv = scales[g.n_kv_heads + h];
   const int64_t hq = row % g.n_q_heads;
-  const float *pp = part + (hq * ((int64_t)g.n_blk + g.n_seqs) + x0 + b) * (2 + D);
+  const float *pp = part + (hq * ((int64_t)g.n_run + g.n_seqs) + x0 + b) * (2 + D);
   float M = -INFINITY, L = 0.0f, A = 0.0f;
   for (int base = 0; base < n_live; base += 64) {
     const int cnt = min(64, n_live - base);
@@ -885,7 +974,8 @@ static bool att_dim_ok(int32_t head_dim) { return head_dim == 64 || head_dim == 
 struct AttnPlan {
   bool mfma, whole;
   int32_t group, unit;
-  int64_t n_blk;
+  uint32_t tail;
+  int64_t n_run, n_blk;
 };
 static AttnPlan att_plan(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim, int32_t max_blocks,
                          int32_t page_size) {
@@ -898,12 +988,14 @@ static AttnPlan att_plan(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads, 
   // units of the longest sequence there can be (lengths are int32)
   const int64_t seq_units = ceil_div(std::min((int64_t)max_blocks * page_size, (int64_t)INT32_MAX), p.unit);
   // resident blocks per group, one equal run each: two per CU (registers, and LDS at D = 128),
-  // three where they fit (64 x 2k-8k, D = 64: 65 against 72 us).  More runs than resident
-  // blocks leave a second, partly filled round: 16 x 1k-8k 37 against 31 us at three per CU.
-  // A number of groups that leaves a part of the CUs without a run takes up to four rounds of
-  // shorter ones where those fill the chip by 5% more (152 groups: 3 runs on 456 of 512, or 10
-  // in three rounds: 16 x 1k-8k, 19 heads per kv head, D = 128 371 -> 311 us, D = 64 221 -> 164).
-  const int64_t resident = (p.mfma && head_dim == 64 ? 3LL : 2LL) * num_cus();
+  // three where they fit (64 x 2k-8k, D = 64: 65 against 72 us; one head per block 64 against
+  // 80, 71 heads on one kv head 297 against 337; at D = 256 1,412 against 1,326 the other way).
+  // More runs than resident blocks leave a second, partly filled round: 16 x 1k-8k 37 against
+  // 31 us at three per CU.  A number of groups that leaves a part of the CUs without a run takes
+  // up to four rounds of shorter ones where those fill the chip by 5% more (152 groups: 3 runs
+  // on 456 of 512, or 10 in three rounds: 16 x 1k-8k, 19 heads per kv head, D = 128 371 -> 311
+  // us, D = 64 221 -> 164).
+  const int64_t resident = ((p.mfma ? head_dim == 64 : p.group == 1 && head_dim < 256) ? 3LL : 2LL) * num_cus();
   int64_t slots = std::max<int64_t>(1, resident / groups);
   double per_round = (double)slots;
   for (int64_t rounds = 2; rounds <= 4; ++rounds) {
@@ -913,10 +1005,14 @@ static AttnPlan att_plan(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads, 
       per_round = (double)n / rounds;
     }
   }
-  // one unit per sequence, or sequences of at most 512 positions that fill half the chip as
-  // they are: whole sequences, no partials (32 x 100-500: 10.2 us, in runs 17)
-  p.whole = seq_units == 1 || (seq_units * p.unit <= 512 && n_seqs >= slots / 2);
-  p.n_blk = p.whole ? n_seqs : std::min(seq_units * n_seqs, slots);
+  p.n_run = std::min(seq_units * n_seqs, slots);
+  p.tail = n_seqs >= p.n_run ? std::max<uint32_t>(1, ATT_TAIL_MANY / p.unit) : ATT_TAIL_ONE;
+  // Whole sequences whatever their lengths, without the merge's launch: one unit each, or at
+  // most 512 positions where they fill half the chip (32 x 100-500: 10.2 us, in runs 17), or
+  // so short that att_take_whole() says so anyway (128 x 100-600, 12 heads, D = 64: 26 -> 19).
+  p.whole = seq_units == 1 || (seq_units * p.unit <= 512 && n_seqs >= slots / 2) ||
+            seq_units <= p.tail;
+  p.n_blk = p.whole ? n_seqs : std::max<int64_t>(p.n_run, n_seqs);  // room for either way of dealing
   return p;
 }
 
@@ -926,35 +1022,37 @@ extern "C" size_t zx_paged_attention_decode_workspace_bytes(int32_t n_seqs, int3
       max_blocks <= 0 || page_size <= 0)
     return 0;
   const AttnPlan p = att_plan(n_seqs, n_q_heads, n_kv_heads, head_dim, max_blocks, page_size);
-  return (size_t)(n_q_heads * (p.n_blk + n_seqs) * (2 + head_dim)) * sizeof(float);
+  // partials, then the table (read by 8 bytes: 2 + head_dim is even)
+  return (size_t)(n_q_heads * (p.n_run + n_seqs) * (2 + head_dim)) * sizeof(float) +
+         (n_seqs > 64 ? AttnTable::bytes(n_seqs, p.n_run) : 0);
 }
 
 template <int G, int D>
 static int launch_partial(dim3 grid, hipStream_t st, const uint16_t *q, const AttnGeom &g, const uint8_t *pool,
                           const float *scales, const int32_t *bt, const int32_t *sl, float *part, uint16_t *out,
-                          int32_t *err) {
+                          int32_t *err, void *table) {
   constexpr int TPW = 64 / (D / 16);
   // (D = 64 with several heads: such pages take the matrix-core variant)
   if ((G == 1 || D > 64) && g.page_size % TPW == 0)
-    paged_decode_partial_kernel<G, D, (G == 1 || D > 64)><<<grid, ATT_THREADS, 0, st>>>(q, g, pool, scales, bt, sl, part, out, err);
+    paged_decode_partial_kernel<G, D, (G == 1 || D > 64)><<<grid, ATT_THREADS, 0, st>>>(q, g, pool, scales, bt, sl, part, out, err, table);
   else
-    paged_decode_partial_kernel<G, D, false><<<grid, ATT_THREADS, 0, st>>>(q, g, pool, scales, bt, sl, part, out, err);
+    paged_decode_partial_kernel<G, D, false><<<grid, ATT_THREADS, 0, st>>>(q, g, pool, scales, bt, sl, part, out, err, table);
   return check_launch("paged_decode_partial");
 }
 
 template <int D>
 static int launch_g(const AttnPlan &p, dim3 grid, hipStream_t st, const uint16_t *q, const AttnGeom &g,
                     const uint8_t *pool, const float *scales, const int32_t *bt, const int32_t *sl, float *part,
-                    uint16_t *out, int32_t *err) {
+                    uint16_t *out, int32_t *err, void *table) {
   if constexpr (D <= 128)
     if (p.mfma) {
-      paged_decode_mfma_kernel<D><<<grid, ATT_THREADS, 0, st>>>(q, g, pool, scales, bt, sl, part, out, err);
+      paged_decode_mfma_kernel<D><<<grid, ATT_THREADS, 0, st>>>(q, g, pool, scales, bt, sl, part, out, err, table);
       return check_launch("paged_decode_mfma");
     }
   switch (p.group) {
-    case 1: return launch_partial<1, D>(grid, st, q, g, pool, scales, bt, sl, part, out, err);
-    case 2: return launch_partial<2, D>(grid, st, q, g, pool, scales, bt, sl, part, out, err);
-    default: return launch_partial<4, D>(grid, st, q, g, pool, scales, bt, sl, part, out, err);
+    case 1: return launch_partial<1, D>(grid, st, q, g, pool, scales, bt, sl, part, out, err, table);
+    case 2: return launch_partial<2, D>(grid, st, q, g, pool, scales, bt, sl, part, out, err, table);
+    default: return launch_partial<4, D>(grid, st, q, g, pool, scales, bt, sl, part, out, err, table);
   }
 }
 
@@ -986,7 +1084,8 @@ extern "C" int zx_paged_attention_decode(const uint16_t *q, int32_t n_q_heads, c
   g.page_size = page_size;
   g.max_blocks = max_blocks;
   g.n_seqs = n_seqs;
-  g.n_blk = (int32_t)p.n_blk;
+  g.n_run = (int32_t)p.n_run;
+  g.tail = p.tail;
   g.unit = (uint32_t)p.unit;
   g.cap = (uint32_t)std::min((int64_t)max_blocks * page_size, (int64_t)INT32_MAX);
   g.whole = p.whole ? 1 : 0;
@@ -1001,17 +1100,25 @@ extern "C" int zx_paged_attention_decode(const uint16_t *q, int32_t n_q_heads, c
   }
   const int64_t gy = n_q_heads / p.group;
   if (gy > 65535) return fail(ZX_ERR_UNSUPPORTED, "paged_attention_decode: too many heads");
+  ZX_REQUIRE(p.n_blk * gy < (1LL << 31), "paged_attention_decode: too many sequences or heads");
+  g.n_group = (int32_t)gy;
   hipStream_t st = as_stream(stream);
   float *part = static_cast<float *>(workspace);
-  const dim3 grid((unsigned)g.n_blk, (unsigned)gy);
+  void *table = part + n_q_heads * (p.n_run + n_seqs) * (2 + head_dim);
+  if (n_seqs > 64 && !p.whole) {
+    paged_decode_plan_kernel<<<1, AP_THREADS, 0, st>>>(g, seq_lens, table);
+    const int prc = check_launch("paged_decode_plan");
+    if (prc) return prc;
+  }
+  const dim3 grid((unsigned)(p.n_blk * gy));
   int rc;
   switch (head_dim) {
-    case 64: rc = launch_g<64>(p, grid, st, q, g, pool, scales, block_tables, seq_lens, part, out, err); break;
-    case 128: rc = launch_g<128>(p, grid, st, q, g, pool, scales, block_tables, seq_lens, part, out, err); break;
-    default: rc = launch_g<256>(p, grid, st, q, g, pool, scales, block_tables, seq_lens, part, out, err); break;
+    case 64: rc = launch_g<64>(p, grid, st, q, g, pool, scales, block_tables, seq_lens, part, out, err, table); break;
+    case 128: rc = launch_g<128>(p, grid, st, q, g, pool, scales, block_tables, seq_lens, part, out, err, table); break;
+    default: rc = launch_g<256>(p, grid, st, q, g, pool, scales, block_tables, seq_lens, part, out, err, table); break;
   }
   if (rc || p.whole) return rc;  // every row is written
   paged_decode_combine_kernel<<<(unsigned)((int64_t)n_seqs * n_q_heads), head_dim, 0, st>>>(part, g, scales, seq_lens,
-                                                                                            out);
+                                                                                            out, table);
   return check_launch("paged_decode_combine");
 }
