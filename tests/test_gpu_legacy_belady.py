@@ -188,3 +188,32 @@ def test_next_use_matches_oracle(dev):
     wnu, wpu = O.next_use(ring, 2 * 8 * 16)
     np.testing.assert_array_equal(nu.cpu().numpy(), wnu)
     np.testing.assert_array_equal(pu.cpu().numpy(), wpu)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n_slabs,slab", [(513, 40_000), (700, 10_001), (767, 33_000), (768, 33_000)])
+def test_int8_legacy_many_slabs(dev, dt, n_slabs, slab):
+    """Slab counts for which one block per slab would leave the CUs uneven: every slab as the
+    per-tensor function gives it."""
+    g = torch.Generator(device=dev).manual_seed(n_slabs)
+    x = (torch.randn((n_slabs, slab), generator=g, device=dev) *
+         torch.logspace(-3, 3, n_slabs, device=dev)[:, None]).to(dt)
+    q, s = kv.int8_legacy_quant_slabs(x)
+    for i in (0, 1, n_slabs // 2, n_slabs - 1):
+        qi, si = kv.int8_legacy_quant(x[i].clone())
+        assert torch.equal(q[i], qi) and torch.equal(s[i], si)
+
+
+def test_int8_legacy_slab_counts_around_two_per_cu(dev):
+    """Two slabs more than two per CU take about as long as two slabs fewer (a quarter longer
+    with one block per slab from there on)."""
+    from test_gpu_attention import least_us
+
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    took = {}
+    for n in (2 * cus - 2, 2 * cus + 2) * 2:
+        x = torch.randn((n, 131072), device=dev)
+        took[n] = min(took.get(n, 1e9), least_us(lambda: kv.int8_legacy_quant_slabs(x)))  # noqa: B023
+    few, many = (took[n] for n in (2 * cus - 2, 2 * cus + 2))
+    print(f"{few:.0f} us, {many:.0f} us", flush=True)
+    assert many <= 1.12 * few

@@ -840,12 +840,17 @@ unsigned legacy_blocks_per_slab(int64_t n_slabs, int64_t slab_len) {
 // blocks per CU hold all rounds (16 Mi bf16 elements, 2,048 rounds: quantised in 18.5 us
 // against 20.0 with half the blocks), else half as many persistent ones, whose maxima the
 // quantiser's every block reads (72 Mi bf16: 60 against 63 us; 16 Mi fp32: 28.9 against 30.9).
+// A number of slabs for which that leaves fewer than three blocks per CU takes more (600 slabs
+// of 131,072 fp32 elements, one block each: 131 us, 118 so).
 constexpr int LEGACY_AMAX_BPC = 8;
+int64_t legacy_amax_most(int64_t n_slabs) { return ceil_div((int64_t)num_cus() * LEGACY_AMAX_BPC, n_slabs); }
 template <int DT> unsigned legacy_amax_blocks(int64_t n_slabs, int64_t slab_len) {
   const int64_t rounds = std::max<int64_t>(1, ceil_div(slab_len / LegacyVec<DT>::W, 256LL * LEGACY_U));
   const int64_t slots = (int64_t)num_cus() * LEGACY_AMAX_BPC;
-  return (unsigned)(rounds <= slots / n_slabs ? rounds
-                                              : std::min(rounds, std::max<int64_t>(1, slots / 2 / n_slabs)));
+  if (rounds <= slots / n_slabs) return (unsigned)rounds;
+  int64_t blocks = std::max<int64_t>(1, slots / 2 / n_slabs);
+  if (blocks * n_slabs < 3LL * num_cus()) blocks = legacy_amax_most(n_slabs);
+  return (unsigned)std::min(rounds, blocks);
 }
 
 size_t legacy_amax_bytes(int64_t n_slabs, int64_t blocks_per_slab) {
@@ -944,7 +949,7 @@ extern "C" int zx_int8_legacy_quant(const void *x, int dtype, int64_t n, int8_t 
 
 extern "C" size_t zx_int8_legacy_quant_slabs_workspace_bytes(int64_t n_slabs) {
   // a word per block of the amax pass
-  return n_slabs > 0 ? legacy_amax_bytes(n_slabs, std::max<int64_t>(1, (int64_t)num_cus() * LEGACY_AMAX_BPC / n_slabs)) : 0;
+  return n_slabs > 0 ? legacy_amax_bytes(n_slabs, legacy_amax_most(n_slabs)) : 0;
 }
 
 extern "C" int zx_int8_legacy_quant_slabs(const void *x, int dtype, int64_t n_slabs, int64_t slab_len, int8_t *q,
