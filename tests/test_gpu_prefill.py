@@ -715,7 +715,7 @@ def test_wide_prefill_weights_far_below_the_largest(below):
     (32, 8, 16, [5, 1, 40], [1500, 600, 2100], True, "f16"),   # several parts; sequences of different lengths
     (8, 2, 16, [33], [1023], True, "exact"),                   # a part per 8 steps, tiles of 32 rows and 1
     (4, 4, 48, [130, 3], [2000, 12], True, "bf16"),            # one head per KV head; a sequence with keys for one part
-    (6, 3, 32, [17, 64], [0, 900], False, "f16"),              # every row sees every key
+    (6, 3, 32, [17, 64], [0, 1500], False, "f16"),             # two heads per KV head; every row sees every key
 ])
 def test_prefill_in_parts(Hq, Hkv, P, n_q, q_pos0, causal, precision):
     """Calls with few query tiles: several blocks share a tile's keys and their parts are
@@ -729,8 +729,9 @@ def test_prefill_in_parts(Hq, Hkv, P, n_q, q_pos0, causal, precision):
     sm = float(np.float32(1.0 / np.sqrt(128)))
     for ranges in ([(lens * r // 3, lens * (r + 1) // 3) for r in range(3)], [(lens * 0 + 3, lens // 3), (lens // 2, lens)]):
         kb, ke = (t(np.array([r[i] for r in ranges], np.int32)) for i in (0, 1))
-        got = kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, kb, ke, causal=causal, sm_scale=sm, check=True,
-                                      precision=precision)
+        got, names = kernels_of(lambda: kv.paged_attention_ring(q, t(cu), t(qp), pool, scales, bt, kb, ke, causal=causal,  # noqa: B023
+                                                                sm_scale=sm, check=True, precision=precision))
+        assert "prefill_combine_kernel" in names
         want, vmax = _f64_rows(q, pool, scales, bt, cu, qp, ranges, causal, sm)
         assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy(), precision)
     zero, end = t(np.zeros(len(n_q), np.int32)), t(lens.astype(np.int32))
