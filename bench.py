@@ -767,7 +767,8 @@ def ring_attention_leg(torch, dev, steps, warmup, skip_cpu):
     out = torch.empty_like(q)
     flops = 4.0 * B * Hq * D * (T * (T + 1) / 2)  # QK^T and PV over the causal (row, key) pairs
     res = {"workload": "ring attention from FP8 pages: 4 seqs x 8192 tokens causal, 32 query heads over 8 KV "
-                       "heads, D=128, page 16 (Llama-3-8B attention shape); kernel paged_prefill_mfma",
+                       "heads, D=128, page 16 (Llama-3-8B attention shape); kernel paged_prefill_wide (one launch, "
+                       "f16 and bf16 P), paged_prefill_mfma (exact, launches)",
            "useful_flop_per_step": flops,
            "note": "peak: the 2.5 PFLOP/s dense bf16/fp16 MFMA figure; with precision 'exact' P.V runs twice "
                    "(P as bf16 hi + lo), so the matrix cores execute 1.5x the useful flops"}
@@ -1139,7 +1140,7 @@ def main():
                         "dtype": "bf16", "config": {"workload": r["workload"]},
                         "roofline": {"bound": "mfma", "achieved": r["ring1"]["TFLOPs"],
                                      "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": r["ring1"]["frac"],
-                                     "traffic": None, "kernel": "paged_prefill_mfma_kernel<4>"}})
+                                     "traffic": None, "kernel": "paged_prefill_wide_kernel"}})
             if "cpu_baseline" in r:
                 out["cpu_baseline"] = r["cpu_baseline"]
 

@@ -234,7 +234,8 @@ int zx_kv_gather_dequant(const uint8_t *pool, int64_t n_pages, int32_t n_heads, 
  * bf16: within 1 bf16 ulp of the same expression evaluated exactly.  A sequence of length
  * 0 gives zeros; rows with an out-of-range page id or a position past max_blocks*P are
  * left out and flagged in *err.  out: [n_seqs][n_q_heads][head_dim] bf16.  workspace:
- * zx_paged_attention_decode_workspace_bytes() device bytes (per-split partial results). */
+ * zx_paged_attention_decode_workspace_bytes() device bytes (partial results, and from 65
+ * sequences on the table of how they are dealt; 0 for a head_dim that is not supported). */
 size_t zx_paged_attention_decode_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads,
                                                  int32_t head_dim, int32_t max_blocks, int32_t page_size);
 int zx_paged_attention_decode(const uint16_t *q, int32_t n_q_heads, const uint8_t *pool, int64_t n_pages,
@@ -389,7 +390,8 @@ int zx_ring_curriculum_trace(const int32_t *degrees, const int32_t *ctx_pages, i
  * NaN codes (e4m3 0x7F / 0xFF): a NaN K element makes the rows that see its key NaN in
  * every channel (lse2 -inf); a NaN V element makes its channel NaN in the rows that see
  * its key, and may also do so in rows before the key whose 64-key step holds it (the
- * product of the step multiplies their weight 0 by the NaN); a merge keeps a NaN of an
+ * product of the step multiplies their weight 0 by the NaN: rows of the 32-row tiles that
+ * reach the step); a merge keeps a NaN of an
  * earlier step. */
 enum {
   ZX_PREFILL_MERGE = 1,
@@ -435,8 +437,8 @@ int zx_paged_attention_ring(const uint16_t *q, int64_t n_q, const int32_t *cu_q,
 
 /* zx_paged_attention_ring with room for partial results (ABI version 8): a call with few
  * query tiles (a chunk of a prompt, a few speculative tokens) whose rows go to out as bf16
- * without merging lets several blocks share a tile's keys and combines their parts, within
- * the tolerance of a ring's steps.  workspace: zx_paged_attention_ring_workspace_bytes()
+ * without merging lets several blocks share a tile's keys (as many as its real number of
+ * keys needs) and combines their parts, within the tolerance of a ring's steps.  workspace: zx_paged_attention_ring_workspace_bytes()
  * device bytes (16-byte aligned) for the same arguments; 0 when the call is not cut, and a
  * smaller or NULL workspace runs it uncut.  n_ranges = 1 is one range per sequence. */
 size_t zx_paged_attention_ring_workspace_bytes(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int32_t page_size,

@@ -740,15 +740,16 @@ __global__ void __launch_bounds__(PF_THREADS, 2) paged_prefill_mfma_kernel(Prefi
 // The same problem for large prefills that write their rows as bf16 (no running output):
 // 64 query rows per wave (two groups of 32), 32x32x16 matrix tiles, one wave per SIMD with
 // the registers of two.  The kernel above is bound by latencies that two waves per SIMD do
-// not hide and reads every K/V operand from LDS for 32 rows (LDS active 58% of the cycles);
-// with 64 rows the operand traffic halves, and one instruction stream is laid out by hand:
+// not hide and reads every K/V operand from LDS for 32 rows (LDS active 56% of the cycles, 21%
+// here); with 64 rows the operand traffic halves, and one instruction stream is laid out by
+// hand:
 //   * S^T of step j (32 matrix instructions) beside the decode and store of step j + 1's K
 //     and V and the weights of the step's first 32 keys;
 //   * P.V of step j - 1 beside the weights of the last 32 keys and the packing of P, each
 //     chunk of P right after the products that read its predecessor.
-// A matrix instruction leaves the vector unit about half of its time, so the two kinds of
-// work add up to what the vector unit can issue (a step of 64 keys: ~2,000 + ~2,000 cycles
-// measured for the two halves, 1,107 + 1,107 of them matrix time).
+// Counters of 4 x 8,192 causal (2.16 ms): matrix cores busy 43% of the SIMD cycles, vector
+// instructions issued in 42%, waits 27%; a step of 64 keys takes about 4,800 cycles, start and
+// end of a block included, 2,048 of them matrix time.
 // No running maximum is computed in these steps: the weights are taken under the maxima the
 // rows have, and only if a lane's sum of 16 weights exceeds 2^PF_LAZY (a score has outgrown
 // its maximum by PF_LAZY, or many have by 4 and more), or where masks apply or a row has no
@@ -1391,17 +1392,19 @@ PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int
     return std::min(ceil_div(max_q_per_seq, qt) * n_seqs, ceil_div(n_q, qt) + n_seqs) * (n_q_heads / p.G);
   };
   // 64 rows per wave where nothing is merged, four query heads share a KV head, there is a
-  // block per CU and contexts can be long: its blocks start and end more slowly (3 x 500-2,000
-  // rows of new sequences: 102 against 90 us; 4 x 512 rows on 8,192 cached: 329 against 346),
-  // one or two heads per KV head gained nothing (2 x 4,096: 150 against 140, 175 against 175),
-  // and the exact mode's second set of weights does not fit its registers.
+  // block per CU and contexts can be long: its blocks start and end more slowly, which shows on
+  // few keys (2 x 4,096 rows on 300: 97 against 86 us; not with a causal mask: 3 x 500-2,000
+  // rows of new sequences 80 against 115, 4 x 512 rows on 8,192 cached 275 against 300).  One
+  // or two heads per KV head gained nothing (2 x 4,096: 150 against 140, 175 against 175), and
+  // the exact mode's second set of weights does not fit its registers.
   p.wide = p.G == 4 && rows_only && p.pm != PF_P_EXACT && cap >= 4096 && blocks(PW_ROWS) >= num_cus();
-  // Few blocks: several share a tile's keys (2 x 300-700 rows on 4k-12k cached 467 -> 254 us,
-  // 256 rows on 16k 443 -> 134, 4 x 4-8 rows on 4k-8k 322 -> 59).  One round of resident blocks
-  // where that gives at least four parts a tile (256 rows on 16k: 169 us with two rounds, whose
-  // parts cost more to combine), else two, which even out sequences of different lengths (2 x
-  // 300-700: 290 us with one); at least 8 steps each (1,024 rows of a new sequence: 56 us in
-  // parts of 4 to 8 steps against 45).
+  // Few blocks: several share a tile's keys (2 x 300-700 rows on 4k-12k cached 467 -> 229 us,
+  // 256 rows on 16k 436 -> 103, 4 x 4-8 rows on 4k-8k 397 -> 50).  One round of resident blocks
+  // where that gives at least four parts a tile, else two, which even out sequences of
+  // different lengths; at least 8 steps each by the table's width.  (These lines were drawn
+  // while one block combined a tile: 256 rows on 16k 169 us with two rounds against 134, 2 x
+  // 300-700 290 with one against 254, 1,024 rows of a new sequence 56 in parts of 4 to 8 steps
+  // against 45.)
   p.n_split = 1;
   const int64_t nb = blocks(32 * 4 / p.G), slots = 2LL * num_cus();
   if (rows_only && !p.wide && nb > 0) {
