@@ -216,4 +216,4 @@ def test_int8_legacy_slab_counts_around_two_per_cu(dev):
         took[n] = min(took.get(n, 1e9), least_us(lambda: kv.int8_legacy_quant_slabs(x)))  # noqa: B023
     few, many = (took[n] for n in (2 * cus - 2, 2 * cus + 2))
     print(f"{few:.0f} us, {many:.0f} us", flush=True)
-    assert many <= 1.12 * few
+    assert many <= 1.15 * few

@@ -779,7 +779,7 @@ def test_parts_follow_the_lengths(Hq, n_q, q_pos0, causal):
         took[name] = min(took.get(name, 1e9), least_us(graph.replay) / 10)
         assert_precision(bits16(out), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy())
     print(f"exact table {took['exact']:.1f} us, 32k table {took['wide']:.1f} us", flush=True)
-    assert took["wide"] <= 1.1 * took["exact"] + 6
+    assert took["wide"] <= 1.1 * took["exact"] + 8
 
 
 @pytest.mark.parametrize("ring", [8, 64])
