@@ -579,6 +579,25 @@ def test_wide_prefill(case, precision):
     assert_precision(bits16(got), bits16(want.to(torch.bfloat16)), vmax.cpu().numpy(), precision)
 
 
+@pytest.mark.parametrize("B,n,old,kernel", [
+    (64, 32, 0, "mfma"), (32, 40, 4000, "mfma"), (64, 256, 0, "mfma"), (24, 600, 0, "mfma"),
+    (4, 512, 0, "wide"), (10, 768, 0, "wide"), (32, 1024, 0, "wide"), (2, 1100, 900, "wide"),
+])
+def test_prefill_kernel_by_rows(B, n, old, kernel):
+    """The 64-row kernel is for calls whose sequences have rows enough for its tiles, whatever
+    the width of the table; others keep the 32-row kernel (64 sequences of 32 rows took 1.6
+    times as long in half-empty tiles, short new sequences up to 1.3 times)."""
+    Hq, Hkv, P = 32, 8, 16
+    q, pool, scales, bt, cu, qp = make(Hq, Hkv, P, [n] * B, [old] * B, [old + n] * B, seed=84)
+    wide_bt = np.zeros((B, 8192 // P), np.int32)
+    wide_bt[:, :bt.shape[1]] = bt
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(DEV)  # noqa: E731
+    args = (q.to(DEV), t(cu), t(qp), t(pool), t(scales), t(wide_bt), t(np.zeros(B, np.int32)),
+            t(np.full(B, old + n, np.int32)))
+    _, names = kernels_of(lambda: kv.paged_attention_prefill(*args, max_q_per_seq=n, check=True))
+    assert f"paged_prefill_{kernel}_kernel" in names
+
+
 def test_wide_prefill_flags_rows_beyond_max_q_per_seq():
     """As test_prefill_flags_rows_beyond_max_q_per_seq, for the 64-row kernel, whose last tile
     would hold 32 rows more: the rows up to a multiple of 32 are computed (as by the 32-row

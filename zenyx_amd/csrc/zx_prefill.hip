@@ -1392,12 +1392,18 @@ PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int
     return std::min(ceil_div(max_q_per_seq, qt) * n_seqs, ceil_div(n_q, qt) + n_seqs) * (n_q_heads / p.G);
   };
   // 64 rows per wave where nothing is merged, four query heads share a KV head, there is a
-  // block per CU and contexts can be long: its blocks start and end more slowly, which shows on
-  // few keys (2 x 4,096 rows on 300: 97 against 86 us; not with a causal mask: 3 x 500-2,000
-  // rows of new sequences 80 against 115, 4 x 512 rows on 8,192 cached 275 against 300).  One
-  // or two heads per KV head gained nothing (2 x 4,096: 150 against 140, 175 against 175), and
-  // the exact mode's second set of weights does not fit its registers.
-  p.wide = p.G == 4 && rows_only && p.pm != PF_P_EXACT && cap >= 4096 && blocks(PW_ROWS) >= num_cus();
+  // block per CU and contexts can be long.  Its blocks start and end more slowly, one to a CU,
+  // so sequences need rows enough: 900 on average, or 320 where four rounds of blocks hold the
+  // call.  (The host does not know the keys; new sequences have the fewest.  Tables of 8,192
+  // positions, 32 rows against 64: 256 x 100 rows 213 us, 239; 64 x 256 150, 184; 25 x 630 188,
+  // 200; 16 x 1,000 245, 240; 23 x 2,048 1,118, 1,014; in four rounds 16 x 250 52, 47; 21 x 380
+  // 88, 88; 10 x 768 115, 105.  With 32 rows and fewer half of a tile is empty: 64 x 32 on 4k-8k
+  // 300, 487.  Few keys without a mask are not kept out: 2 x 4,096 rows on 300 86, 97.)  One or
+  // two heads per KV head gained nothing (2 x 4,096: 150 against 140, 175 against 175), and the
+  // exact mode's second set of weights does not fit its registers.
+  const int64_t wide_blocks = blocks(PW_ROWS), rows = n_q / n_seqs;
+  p.wide = p.G == 4 && rows_only && p.pm != PF_P_EXACT && cap >= 4096 && wide_blocks >= num_cus() &&
+           (rows >= 900 || (rows >= 320 && wide_blocks <= 4LL * num_cus()));
   // Few blocks: several share a tile's keys (2 x 300-700 rows on 4k-12k cached 467 -> 229 us,
   // 256 rows on 16k 436 -> 103, 4 x 4-8 rows on 4k-8k 397 -> 50).  One round of resident blocks
   // where that gives at least four parts a tile, else two, which even out sequences of
