@@ -247,3 +247,21 @@ def test_prefill_plan_under_a_loose_bound():
         assert tight > 0
         for most in (n_q + 1, 131072, 2**31 - 1):
             assert size(n_q, Hq, Hkv, 16, 600, n_seqs, most, 1, N.ZX_PREFILL_BF16) == tight
+
+
+def test_prefill_is_not_cut_where_its_tiles_fill_the_chip():
+    """Two parts a tile only cost where the uncut tiles take one full round of blocks (two per
+    CU; 256 CUs where there is no device)."""
+    from zenyx_amd import _native as N
+
+    size = N.load().zx_paged_attention_ring_workspace_bytes
+    cus = 256
+    try:
+        import torch
+        if torch.cuda.is_available():
+            cus = torch.cuda.get_device_properties(0).multi_processor_count
+    except RuntimeError:
+        pass
+    tiles = 2 * cus // 8  # sequences of one tile for 8 head groups
+    for n_seqs, cut in ((tiles, False), (tiles * 15 // 16, False), (tiles * 3 // 4, True), (tiles // 4, True)):
+        assert (size(32 * n_seqs, 32, 8, 16, 512, n_seqs, 32, 1, N.ZX_PREFILL_BF16) > 0) == cut, n_seqs

@@ -1407,15 +1407,17 @@ PrefillPlan prefill_plan(int64_t n_q, int32_t n_q_heads, int32_t n_kv_heads, int
   // Few blocks: several share a tile's keys (2 x 300-700 rows on 4k-12k cached 467 -> 229 us,
   // 256 rows on 16k 436 -> 103, 4 x 4-8 rows on 4k-8k 397 -> 50).  One round of resident blocks
   // where that gives at least four parts a tile, else two, which even out sequences of
-  // different lengths; at least 8 steps each by the table's width.  (These lines were drawn
-  // while one block combined a tile: 256 rows on 16k 169 us with two rounds against 134, 2 x
-  // 300-700 290 with one against 254, 1,024 rows of a new sequence 56 in parts of 4 to 8 steps
-  // against 45.)
+  // different lengths; none where the tiles fill the round as they are (64 x 32 rows on 6,000
+  // cached 254 against 279 us in two parts, 32 x 64 on 4k-8k 299 against 325; 16 x 128 on
+  // 500-16k the other way, 481 against 366); at least 8 steps each by the table's width.  (The
+  // other lines were drawn while one block combined a tile: 256 rows on 16k 169 us with two
+  // rounds against 134, 2 x 300-700 290 with one against 254, 1,024 rows of a new sequence 56 in
+  // parts of 4 to 8 steps against 45.)
   p.n_split = 1;
   const int64_t nb = blocks(32 * 4 / p.G), slots = 2LL * num_cus();
   if (rows_only && !p.wide && nb > 0) {
     const int64_t steps = (cap - (causal ? std::min<int64_t>(max_q_per_seq, cap) / 2 : 0)) / PF_KEYS;
-    const int64_t parts = slots / nb >= 4 ? slots / nb : 2 * slots / nb;
+    const int64_t parts = slots / nb >= 4 ? slots / nb : (nb * 8 > slots * 7 ? 1 : 2 * slots / nb);
     p.n_split = (int)std::max<int64_t>(1, std::min({parts, steps / 8, (int64_t)PC_MAX}));
   }
   p.QT = p.wide ? PW_ROWS : 32 * 4 / p.G;
